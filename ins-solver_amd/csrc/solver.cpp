@@ -20,6 +20,12 @@ enum : int {
 static_assert(S_BNUM == S_RZN + 1, "dot_rz_flex writes r.z and r.(z - zold) to adjacent slots");
 
 int64_t round_up(int64_t v, int64_t m) { return ((v + m - 1) / m) * m; }
+
+// Two vectors of n doubles that share no entry.
+bool disjoint(const double* a, const double* b, size_t n) {
+  const uintptr_t x = reinterpret_cast<uintptr_t>(a), y = reinterpret_cast<uintptr_t>(b);
+  return x + n * sizeof(double) <= y || y + n * sizeof(double) <= x;
+}
 }  // namespace
 
 template <typename T>
@@ -335,23 +341,45 @@ void PoissonSolver::grad_central(const double* p, double* const g[3], const doub
     lift_.upload(lift.data(), lift.size());
   }
   const size_t n = (size_t)Np * stride_;
-  DBuf<double> pd;
-  pd.alloc(n);
-  import_vec(p, pd.p, layout, Np);
-  DBuf<double> ud[3], od[3];
+  const Level& l0 = *levels_[0];
+  // The caller's own vectors where they have the solver's layout and no output overlaps an input
+  // that other threads still read: an output may be its own uT component, entry by entry.
+  bool direct = layout == Layout::DEVICE_SOA && dat_stride() == stride_;
+  for (int x = 0; x < d && direct; ++x) {
+    direct = disjoint(g[x], p, n);
+    for (int y = 0; y < d; ++y) {
+      if (y != x) direct = direct && disjoint(g[x], g[y], n);
+      if (u && u[y] && !(y == x && u[y] == g[x])) direct = direct && disjoint(g[x], u[y], n);
+    }
+  }
+  if (u)
+    for (int x = 0; x < d; ++x)
+      if (!u[x]) throw InvalidArgument("null velocity component");
   const double* up[3] = {nullptr, nullptr, nullptr};
   double* op[3] = {nullptr, nullptr, nullptr};
+  if (direct) {
+    for (int x = 0; x < d; ++x) {
+      op[x] = g[x];
+      if (u) up[x] = u[x];
+    }
+    launch_grad_central(d, N_, E, stride_, grad_xi_.p, nbr_.p, code_.p, l0.C64.p, l0.tab.p, lift_.p, p, dt,
+                        up, op, stream_);
+    INSP_HIP(hipStreamSynchronize(stream_));
+    return;
+  }
+  DBuf<double> pd;
+  pd.alloc(n, false);  // import_vec and the kernel write whole rows, padding included
+  import_vec(p, pd.p, layout, Np);
+  DBuf<double> ud[3], od[3];
   for (int x = 0; x < d; ++x) {
-    od[x].alloc(n);
+    od[x].alloc(n, false);
     op[x] = od[x].p;
     if (u) {
-      if (!u[x]) throw InvalidArgument("null velocity component");
-      ud[x].alloc(n);
+      ud[x].alloc(n, false);
       import_vec(u[x], ud[x].p, layout, Np);
       up[x] = ud[x].p;
     }
   }
-  const Level& l0 = *levels_[0];
   launch_grad_central(d, N_, E, stride_, grad_xi_.p, nbr_.p, code_.p, l0.C64.p, l0.tab.p, lift_.p, pd.p,
                       dt, up, op, stream_);
   for (int x = 0; x < d; ++x) export_vec(od[x].p, g[x], layout, Np);
