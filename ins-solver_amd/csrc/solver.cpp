@@ -1452,25 +1452,41 @@ int PoissonSolver::solve(const double* rhs, double* ans, Layout layout, SolveSta
 
 void PoissonSolver::mult(const double* in, double* out, Layout layout, bool fp32) {
   if (!initialised_) init();
-  const int64_t n = (int64_t)np() * stride_;
-  import_vec(in, b_.p, layout, np());
+  const size_t n = (size_t)np() * stride_;
+  const int64_t E = mesh_.n_cells;
+  // The caller's own vectors where they have the solver's layout: the passes read cells only, so
+  // the input's padding may hold anything; the output's is cleared.
+  const bool own = layout == Layout::DEVICE_SOA && dat_stride() == stride_ && in && out;
   if (!fp32) {
-    apply_level<double>(0, b_.p, Ap_.p);
-  } else {
-    Level& l0 = *levels_[0];
-    DBuf<float> xf, yf;
-    xf.alloc(n);
-    yf.alloc(n);
-    if (var_factor_ && l0.w32.k.empty()) {
-      l0.w32.k.alloc(n);
-      convert<double, float>(n, l0.w64.k.p, l0.w32.k.p, stream_);
+    if (own && disjoint(in, out, n)) {
+      apply_level<double>(0, in, out);
+      zero_padding<double>(np(), E, stride_, out, stream_);
+    } else {
+      import_vec(in, b_.p, layout, np());
+      apply_level<double>(0, b_.p, Ap_.p);
+      export_vec(Ap_.p, out, layout, np());
     }
-    convert<double, float>(n, b_.p, xf.p, stream_);
-    apply_level<float>(0, xf.p, yf.p);
-    convert<float, double>(n, yf.p, Ap_.p, stream_);
     INSP_HIP(hipStreamSynchronize(stream_));
+    return;
   }
-  export_vec(Ap_.p, out, layout, np());
+  Level& l0 = *levels_[0];
+  if (var_factor_ && l0.w32.k.empty()) {
+    l0.w32.k.alloc(n);
+    convert<double, float>((int64_t)n, l0.w64.k.p, l0.w32.k.p, stream_);
+  }
+  // both FP32 vectors live in r_, which every solve writes whole before it reads it
+  float* xf = reinterpret_cast<float*>(r_.p);
+  float* yf = xf + n;
+  const double* src = in;
+  if (!own) {
+    import_vec(in, b_.p, layout, np());
+    src = b_.p;
+  }
+  convert_rows<double, float>(np(), E, stride_, src, xf, stream_);
+  apply_level<float>(0, xf, yf);
+  double* dst = own ? out : Ap_.p;
+  convert_rows<float, double>(np(), E, stride_, yf, dst, stream_);
+  if (!own) export_vec(dst, out, layout, np());
   INSP_HIP(hipStreamSynchronize(stream_));
 }
 

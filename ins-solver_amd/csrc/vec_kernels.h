@@ -95,6 +95,10 @@ void cheb_step3(int64_t n, const T* f, const T* Ax, const T* invdiag, const T* p
 // y = x converted
 template <typename Tin, typename Tout>
 void convert(int64_t n, const Tin* x, Tout* y, hipStream_t s);
+// The same for row vectors (v[i*stride + e], e < E) with the padding of y cleared; x may hold
+// anything in its padding.
+template <typename Tin, typename Tout>
+void convert_rows(int rows, int64_t E, int64_t stride, const Tin* x, Tout* y, hipStream_t s);
 template <typename T>
 void fill(int64_t n, T* x, T v, hipStream_t s);
 template <typename T>
