@@ -6,6 +6,8 @@
 #include <cmath>
 #include <cstring>
 
+#include "split_passes.h"
+
 namespace insp {
 
 namespace {
@@ -149,7 +151,7 @@ PoissonSolver::PoissonSolver(HostMesh mesh, int order, hipStream_t stream)
   std::vector<int> bt((size_t)std::max<int64_t>(mesh_.n_bfaces, 1), 0);
   bctype_.upload(bt.data(), bt.size());
   scal_.alloc(S_COUNT);
-  partial_.alloc((size_t)std::max<int64_t>(4 * kRedBlocks, apply_blocks(E)));
+  partial_.alloc((size_t)std::max<int64_t>(4 * kRedBlocks, split_blocks(E)));
   INSP_HIP(hipHostMalloc((void**)&host_scal_, S_COUNT * sizeof(double), hipHostMallocDefault));
 }
 
@@ -714,7 +716,9 @@ hipEvent_t PoissonSolver::ev_take() {
 }
 
 template <typename T>
-void PoissonSolver::apply_level(int l, const T* u, T* out, double* partial, T* tr, bool cells) {
+int PoissonSolver::apply_level(int l, const T* u, T* out, double* partial, T* tr, bool cells) {
+  bool mass_done = false;
+  int npart = apply_blocks(mesh_.n_cells);
   Level& lv = *levels_[l];
   Work<T>& w = lv.work<T>();
   const bool own_tr = tr == nullptr;  // a caller-given trace buffer: no allocation, no events
@@ -743,12 +747,19 @@ void PoissonSolver::apply_level(int l, const T* u, T* out, double* partial, T* t
   } else if (oi_ && l == 0) {
     if (prof) INSP_HIP(hipEventRecord(e1, stream_));
     launch_apply_oi<T>(mv, v, oi_view<T>(), u, out, stream_, partial);
+  } else if (!v.frag && split_apply(mv, v, std::is_same<T, float>::value)) {
+    trace_pass<T>(mv, v, u, k, tr, stream_);
+    if (prof) INSP_HIP(hipEventRecord(e1, stream_));
+    launch_apply_split<T>(mv, v, u, tr, k, MassView<T>{var_mm_ ? w.mm.p : nullptr, (T)mm_const_}, out,
+                          stream_, partial);
+    mass_done = true;
+    npart = split_blocks(mesh_.n_cells);
   } else {
-    launch_trace<T>(mv, v, u, k, tr, stream_);
+    trace_pass<T>(mv, v, u, k, tr, stream_);
     if (prof) INSP_HIP(hipEventRecord(e1, stream_));
     launch_apply<T>(mv, v, u, tr, k, out, stream_, partial);
   }
-  if (has_mass_term()) {
+  if (has_mass_term() && !mass_done) {
     if (cells) throw std::logic_error("cell-by-cell apply with a mass term");
     launch_mass_add<T>(mv, v, lv.L.Np, var_mm_ ? w.mm.p : nullptr, (T)mm_const_, u, out, stream_,
                        partial);
@@ -761,6 +772,7 @@ void PoissonSolver::apply_level(int l, const T* u, T* out, double* partial, T* t
     INSP_HIP(hipEventRecord(e2, stream_));
     ev_coarse_.push_back({e0, e2});
   }
+  return npart;
 }
 
 CoarseTiming PoissonSolver::take_coarse_timing() {
@@ -830,10 +842,12 @@ void PoissonSolver::chebyshev(int l, const T* f, T* x, bool zero_init) {
     if (fuse) {
       if (w.tr.empty()) w.tr.alloc((size_t)lv.L.Nf * lv.L.Nfp * stride_);
       const T* k = var_factor_ ? w.k.p : nullptr;
-      launch_trace<T>(mv, v, x, k, w.tr.p, stream_);
       const T* prev = prev_zero ? nullptr : w.x2.p;
       prev_zero = false;
-      if (!launch_apply_cheb<T>(mv, v, x, w.tr.p, k, f, w.inv.p, prev, w.x2.p, c1, c2, stream_))
+      trace_pass<T>(mv, v, x, k, w.tr.p, stream_);
+      if (split_apply(mv, v, std::is_same<T, float>::value))
+        launch_cheb_split<T>(mv, v, x, w.tr.p, k, f, w.inv.p, prev, w.x2.p, c1, c2, stream_);
+      else if (!launch_apply_cheb<T>(mv, v, x, w.tr.p, k, f, w.inv.p, prev, w.x2.p, c1, c2, stream_))
         throw std::logic_error("fused Chebyshev step not available on this level");
       std::swap(w.x, w.x2);
       x = w.x.p;
@@ -904,8 +918,8 @@ void PoissonSolver::coarse_cg(int l) {
       apply_level<T>(l, pc, w.Ap.p);
       dot<T>(n, pc, w.Ap.p, nullptr, nullptr, 1, scal_.p, S_CG_PAP, rs, stream_);
     } else {
-      apply_level<T>(l, pc, w.Ap.p, partial_.p, nullptr, cells);  // p.Ap fused into the pass
-      finalize(apply_blocks(mesh_.n_cells), 1, partial_.p, scal_.p, S_CG_PAP, stream_);
+      const int nparts = apply_level<T>(l, pc, w.Ap.p, partial_.p, nullptr, cells);  // p.Ap fused into the pass
+      finalize(nparts, 1, partial_.p, scal_.p, S_CG_PAP, stream_);
     }
     ++smoother_applies_;
     cg_update_z<T>(n, w.z.p, w.Ap.p, inv, scal_.p, a, S_CG_PAP, b, rs, stream_);
@@ -1279,8 +1293,8 @@ int PoissonSolver::fcg_mixed(double tol, int* iters, double* rr_out, int64_t* fi
       apply_level<float>(0, p32_.p, Ap32_.p);
       dot<float>(n, p32_.p, Ap32_.p, nullptr, nullptr, 1, scal_.p, S_PAP, rs, stream_);
     } else {
-      apply_level<float>(0, p32_.p, Ap32_.p, partial_.p);  // p.Ap fused into the element pass
-      finalize(apply_blocks(mesh_.n_cells), 1, partial_.p, scal_.p, S_PAP, stream_);
+      const int nparts = apply_level<float>(0, p32_.p, Ap32_.p, partial_.p);  // p.Ap fused into the element pass
+      finalize(nparts, 1, partial_.p, scal_.p, S_PAP, stream_);
     }
     cg_update_xr_mixed(n, x_.p, r, p32_.p, Ap32_.p, scal_.p, S_RZ, S_PAP, S_RR, rs, stream_);
     ++it;
@@ -1412,9 +1426,9 @@ int PoissonSolver::solve(const double* rhs, double* ans, Layout layout, SolveSta
       copy<double>(n, z_.p, p_.p, stream_);
       bool breakdown = false;
       while (it < max_iter_) {
-        apply_level<double>(0, p_.p, Ap_.p, partial_.p);  // p.Ap fused into the element pass
+        const int nparts = apply_level<double>(0, p_.p, Ap_.p, partial_.p);  // p.Ap fused into the element pass
         ++fine_applies;
-        finalize(apply_blocks(mesh_.n_cells), 1, partial_.p, scal_.p, S_PAP, stream_);
+        finalize(nparts, 1, partial_.p, scal_.p, S_PAP, stream_);
         cg_update_xr<double>(n, x_.p, r, p_.p, Ap_.p, nullptr, nullptr, scal_.p, S_RZ, S_PAP,
                              S_RR, rs, stream_);
         ++it;

@@ -231,8 +231,9 @@ class PoissonSolver {
   void ensure_factor_levels();
   void compute_diagonals();
   void estimate_eigenvalues();
+  // returns the number of partials of u.(A u) that it leaves in `partial`
   template <typename T>
-  void apply_level(int l, const T* u, T* out, double* partial = nullptr, T* tr = nullptr,
+  int apply_level(int l, const T* u, T* out, double* partial = nullptr, T* tr = nullptr,
                    bool cells = false);
   // finest level: coefficient and mass-term factor (null when constant), face nodes per cell
   const double* fine_factor() const;

@@ -5,6 +5,7 @@
 
 #include "kernels.h"
 #include "refelem.h"
+#include "split_passes.h"
 #include "vec_kernels.h"
 
 namespace insp {
@@ -144,7 +145,7 @@ void VecViscousSolver::apply(const double* u, double* out, double* partial) {
   const double* k = base_.fine_factor();
   const int64_t cs = (int64_t)base_.np() * base_.stride_;
   const int64_t ts = (int64_t)base_.fine_face_nodes() * base_.stride_;
-  for (int c = 0; c < ncomp_; ++c) launch_trace<double>(mv, lv, u + c * cs, k, tr_.p + c * ts, base_.stream_);
+  for (int c = 0; c < ncomp_; ++c) trace_pass<double>(mv, lv, u + c * cs, k, tr_.p + c * ts, base_.stream_);
   for (int c = 0; c < ncomp_; ++c) apply_one(c, u, out + c * cs, partial);
 }
 
@@ -200,7 +201,7 @@ void VecViscousSolver::build_block_jacobi() {
     for (int c = 0; c < ncol; ++c)
       for (int j = 0; j < Np; ++j) {
         block_probe_unit(Np, E, st, dcol.p, c, j, u.p + comp * cs, base_.stream_);
-        launch_trace<double>(mv, lv, u.p + comp * cs, k, tr_.p + comp * ts, base_.stream_);
+        trace_pass<double>(mv, lv, u.p + comp * cs, k, tr_.p + comp * ts, base_.stream_);
         apply_one(comp, u.p, y.p, nullptr);
         block_extract_column(Np, E, st, dcol.p, c, j, y.p, blk_.p + comp * bs, base_.stream_);
       }
