@@ -21,7 +21,7 @@ SOURCES = ["refelem.cpp", "mesh.cpp", "hdf5_reader.cpp", "solver.cpp", "viscous_
            "capi.cpp", "sipg_kernels.hip", "vec_kernels.hip", "batch_kernels.hip",
            "amg_kernels.hip", "block_kernels.hip", "rhs_kernels.hip", "sipg_mfma.hip",
            "probe_kernels.hip", "mass_kernels.hip",
-           "proj_kernels.hip", "sipg_oi.hip", "sipg_split.hip",
+           "proj_kernels.hip", "sipg_oi.hip", "sipg_split.hip", "cg_kernels.hip",
            "sipg_split_3d3.hip", "sipg_split_3d4.hip", "sipg_split_3d4f.hip"]
 
 COMMON = ["-O3", "-std=c++17", "-fPIC", f"--offload-arch={ARCH}",

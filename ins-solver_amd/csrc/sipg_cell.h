@@ -360,20 +360,77 @@ struct BitNodes {
   P1NodeBits b;
 };
 
-template <int DIM, typename T, int VAR, bool PACK = false, class Out = T*, class Slip = NoSlip,
-          class Nodes = TabNodes, bool KAOS = false, bool VCM = false>
-__device__ __forceinline__ double
-apply_p1_cell(int64_t e, int64_t stride, const T* __restrict__ u, const double* __restrict__ Kt,
-              const double* __restrict__ tauS, const int* __restrict__ nbr,
-              const int* __restrict__ code, const int* __restrict__ bctype,
-              const T* __restrict__ kfac, cptr<T> __restrict__ C, cptr<int> __restrict__ tab,
-              Out out, const Slip& slip = Slip{}, const Nodes& nodes = Nodes{}) {
+// What the order-1 pass holds of a cell and its neighbours after its loads.
+template <int DIM, typename T>
+struct P1Loads {
+  static constexpr OpLayout L = op_layout(DIM, 1);
+  static constexpr int Np = L.Np, Nfp = L.Nfp, Nf = L.Nf, NK = L.NK;
+  int nb[Nf], c[Nf];                       // neighbour or -(bface+1), its code
+  T uu[Np], kk[Np], K[NK], ts[Nf];         // values, coefficient, metric, penalties
+  T un[Nf][Np], kn[Nf][NK], fn_k[Nf][Np];  // the neighbours' values, metric, coefficient
+  int nd[Nf][Nfp], bt[Nf];                 // neighbour's node at each face node; boundary type
+  // the cell behind face f, or the cell itself
+  __device__ __forceinline__ int64_t at(int f, int64_t e) const { return nb[f] >= 0 ? (int64_t)nb[f] : e; }
+};
+
+// Nodal values of cell q of an order-1 vector: in rows, or (VCM, 3D) cell by cell ([E][Np], 16 or 32
+// bytes per cell).
+template <int Np, bool VCM, typename T>
+__device__ __forceinline__ void p1_values(const T* __restrict__ u, int64_t stride, int64_t q, T* dst) {
+  if constexpr (VCM) {
+    static_assert(Np == 4, "cell-by-cell values: 3D order 1");
+    if constexpr (sizeof(T) == 8) {
+      const double2* uq = reinterpret_cast<const double2*>(u) + q * 2;
+      const double2 a = uq[0], b = uq[1];
+      dst[0] = a.x; dst[1] = a.y; dst[2] = b.x; dst[3] = b.y;
+    } else {
+      const float4 a = reinterpret_cast<const float4*>(u)[q];
+      dst[0] = a.x; dst[1] = a.y; dst[2] = a.z; dst[3] = a.w;
+    }
+  } else {
+#pragma unroll
+    for (int m = 0; m < Np; ++m) dst[m] = u[m * stride + q];
+  }
+}
+
+template <int Np, bool VCM, typename T>
+__device__ __forceinline__ void p1_store(T* o, int64_t stride, int64_t e, const T (&v)[Np]) {
+  if constexpr (VCM) {
+    static_assert(Np == 4, "cell-by-cell values: 3D order 1");
+    if constexpr (sizeof(T) == 8) {
+      double2* oq = reinterpret_cast<double2*>(o) + e * 2;
+      oq[0] = make_double2(v[0], v[1]);
+      oq[1] = make_double2(v[2], v[3]);
+    } else {
+      reinterpret_cast<float4*>(o)[e] = make_float4(v[0], v[1], v[2], v[3]);
+    }
+  } else {
+#pragma unroll
+    for (int m = 0; m < Np; ++m) o[m * stride + e] = v[m];
+  }
+}
+
+// Two-bit field c of w (c < 6 in 2D, < 24 in 3D), by 32-bit shifts: v_lshrrev_b64 with its amount in the
+// last VGPR of the wave's allocation (v79 of 80) took wrong amounts in about one wave of 2000 here
+// (2D order-1 apply, 125,000 cells, other results on every launch).
+template <int DIM>
+__device__ __forceinline__ int node_field(unsigned long long w, int c) {
+  const unsigned lo = (unsigned)w, hi = (unsigned)(w >> 32);
+  if constexpr (DIM == 2) return (int)((lo >> (2 * c)) & 3u);
+  else return (int)(((c < 16 ? lo : hi) >> ((2 * c) & 31)) & 3u);
+}
+
+// Both rounds of loads. VCM: u holds the values, nbr the packed words and tauS the penalties cell by
+// cell ([E][4]); the coefficient stays in rows. KAOS: Kt holds the metric cell by cell ([E][NK]).
+template <int DIM, typename T, int VAR, bool PACK, class Nodes, bool KAOS, bool VCM>
+__device__ __forceinline__ void
+p1_load(int64_t e, int64_t stride, const T* __restrict__ u, const double* __restrict__ Kt,
+        const double* __restrict__ tauS, const int* __restrict__ nbr, const int* __restrict__ code,
+        const int* __restrict__ bctype, const T* __restrict__ kfac, cptr<int> __restrict__ tab,
+        const Nodes& nodes, P1Loads<DIM, T>& P) {
   constexpr OpLayout L = op_layout(DIM, 1);
   constexpr int Np = L.Np, Nfp = L.Nfp, Nf = L.Nf, NK = L.NK;
-  constexpr FmaskTable FM = make_fmask(DIM, 1);
-  // round 1; VCM: nbr holds the packed words and tauS the penalties cell by cell ([E][4])
   static_assert(!VCM || PACK, "cell-by-cell values: packed words");
-  int nb[Nf], c[Nf];
   int wcell[Nf];
   if constexpr (VCM) {
     const int4 w4 = reinterpret_cast<const int4*>(nbr)[e];
@@ -383,39 +440,16 @@ apply_p1_cell(int64_t e, int64_t stride, const T* __restrict__ u, const double* 
   for (int f = 0; f < Nf; ++f) {
     if constexpr (PACK) {
       const int w = VCM ? wcell[f] : nbr[f * stride + e];
-      nb[f] = w >= 0 ? w >> 5 : w;
-      c[f] = w >= 0 ? (w & 31) : 0;
+      P.nb[f] = w >= 0 ? w >> 5 : w;
+      P.c[f] = w >= 0 ? (w & 31) : 0;
     } else {
-      nb[f] = nbr[f * stride + e];
-      c[f] = nb[f] >= 0 ? code[f * stride + e] : 0;
+      P.nb[f] = nbr[f * stride + e];
+      P.c[f] = P.nb[f] >= 0 ? code[f * stride + e] : 0;
     }
   }
-  // VCM: u and out hold the values cell by cell ([E][Np], 3D: 16 or 32 bytes per cell) instead of
-  // in rows; the coefficient stays in rows
-  static_assert(!VCM || Np == 4, "cell-by-cell values: 3D order 1");
-  auto values = [&](int64_t q, T* dst) {
-    if constexpr (VCM) {
-      if constexpr (sizeof(T) == 8) {
-        const double2* uq = reinterpret_cast<const double2*>(u) + q * 2;
-        const double2 a = uq[0], b = uq[1];
-        dst[0] = a.x; dst[1] = a.y; dst[2] = b.x; dst[3] = b.y;
-      } else {
-        const float4 a = reinterpret_cast<const float4*>(u)[q];
-        dst[0] = a.x; dst[1] = a.y; dst[2] = a.z; dst[3] = a.w;
-      }
-    } else {
+  p1_values<Np, VCM>(u, stride, e, P.uu);
 #pragma unroll
-      for (int m = 0; m < Np; ++m) dst[m] = u[m * stride + q];
-    }
-  };
-  T uu[Np], acc[Np], kk[Np];
-  values(e, uu);
-#pragma unroll
-  for (int m = 0; m < Np; ++m) {
-    acc[m] = 0;
-    kk[m] = kval<VAR>(kfac, m * stride + e);
-  }
-  // KAOS: Kt holds the metric cell by cell ([E][NK]) instead of in rows
+  for (int m = 0; m < Np; ++m) P.kk[m] = kval<VAR>(kfac, m * stride + e);
   static_assert(!KAOS || NK % 2 == 0, "the cell-by-cell metric is read in pairs");
   auto metric = [&](int64_t q, T* dst) {
     if constexpr (KAOS) {
@@ -431,44 +465,61 @@ apply_p1_cell(int64_t e, int64_t stride, const T* __restrict__ u, const double* 
       for (int k = 0; k < NK; ++k) dst[k] = (T)Kt[k * stride + q];
     }
   };
-  T K[NK];
-  metric(e, K);
-  T ts[Nf];
+  metric(e, P.K);
   if constexpr (VCM) {
     const double2* tq = reinterpret_cast<const double2*>(tauS) + e * 2;
     const double2 t01 = tq[0], t23 = tq[1];
-    ts[0] = (T)t01.x; ts[1] = (T)t01.y; ts[2] = (T)t23.x; ts[3] = (T)t23.y;
+    P.ts[0] = (T)t01.x; P.ts[1] = (T)t01.y; P.ts[2] = (T)t23.x; P.ts[3] = (T)t23.y;
   } else {
 #pragma unroll
-    for (int f = 0; f < Nf; ++f) ts[f] = (T)tauS[f * stride + e];
+    for (int f = 0; f < Nf; ++f) P.ts[f] = (T)tauS[f * stride + e];
   }
   // round 2
-  T un[Nf][Np], kn[Nf][NK], fn_k[Nf][Np];
-  int nd[Nf][Nfp], bt[Nf];
 #pragma unroll
   for (int f = 0; f < Nf; ++f) {
-    const bool in = nb[f] >= 0;
-    const int64_t q = in ? (int64_t)nb[f] : e;
-    const int cf = in ? c[f] : 0;
-    values(q, un[f]);
+    const bool in = P.nb[f] >= 0;
+    const int64_t q = P.at(f, e);
+    const int cf = in ? P.c[f] : 0;
+    p1_values<Np, VCM>(u, stride, q, P.un[f]);
 #pragma unroll
-    for (int m = 0; m < Np; ++m) fn_k[f][m] = kval<VAR>(kfac, m * stride + q);
-    metric(q, kn[f]);
+    for (int m = 0; m < Np; ++m) P.fn_k[f][m] = kval<VAR>(kfac, m * stride + q);
+    metric(q, P.kn[f]);
 #pragma unroll
     for (int j = 0; j < Nfp; ++j) {
-      if constexpr (std::is_same<Nodes, BitNodes>::value)  // 3D: the same row for every face
-        nd[f][j] = (int)((nodes.b.w[DIM == 3 ? 0 : f][j] >> (2 * cf)) & 3ull);
+      if constexpr (std::is_same<Nodes, BitNodes>::value)
+        P.nd[f][j] = node_field<DIM>(nodes.b.w[DIM == 3 ? 0 : f][j], cf);  // 3D: the same row for every face
       else
-        nd[f][j] = tab[L.tab_nbr + (f * Nf * L.nperm + cf) * Nfp + j] >> 6;
+        P.nd[f][j] = tab[L.tab_nbr + (f * Nf * L.nperm + cf) * Nfp + j] >> 6;
     }
-    bt[f] = in ? 0 : bctype[-nb[f] - 1];
+    P.bt[f] = in ? 0 : bctype[-P.nb[f] - 1];
   }
+}
 
+// The arithmetic: acc = (A u) at the cell's nodes; returns u.(A u) over the cell.
+template <int DIM, typename T, int VAR, class Slip>
+__device__ __forceinline__ double
+p1_compute(int64_t e, int64_t stride, const P1Loads<DIM, T>& P, const Slip& slip,
+           T (&acc)[op_layout(DIM, 1).Np]) {
+  constexpr OpLayout L = op_layout(DIM, 1);
+  constexpr int Np = L.Np, Nfp = L.Nfp, Nf = L.Nf;
+  constexpr FmaskTable FM = make_fmask(DIM, 1);
+  const auto& nb = P.nb;
+  const auto& c = P.c;
+  const auto& uu = P.uu;
+  const auto& kk = P.kk;
+  const auto& K = P.K;
+  const auto& ts = P.ts;
+  const auto& un = P.un;
+  const auto& kn = P.kn;
+  const auto& fn_k = P.fn_k;
+  const auto& nd = P.nd;
+  const auto& bt = P.bt;
+#pragma unroll
+  for (int m = 0; m < Np; ++m) acc[m] = 0;
   // P1: grad phi_i is constant, so Bt[r][j][i] = dphi_ri m_j and Wt[f][r][j][i] = dphi_ri w_j
   // (m, w: column sums of the mass and face mass). The volume term and every face's symmetry
   // term collapse into one vector V: acc_i += sum_r dphi_ri V_r at the end, with
   // V = (sum_j m_j k_j) h + sum_f beta_f sum_j w_j sig_fj.
-  (void)C;
   // c_f: the face mass factor; c_s = -w/2 with the face mass column sum w = c_f (Nfp + 1)
   constexpr T c_m = (T)p1_mass_colsum(DIM), c_f = (T)p1_face_mass_c(DIM),
               c_s = (T)(-0.5 * p1_face_mass_c(DIM) * (Nfp + 1));
@@ -589,23 +640,34 @@ apply_p1_cell(int64_t e, int64_t stride, const T* __restrict__ u, const double* 
 #pragma unroll
     for (int r = 0; r < DIM; ++r) acc[r + 1] = fma((T)0.5, V[r], acc[r + 1]);
   }
-  if constexpr (VCM) {
-    static_assert(std::is_same<Out, T*>::value, "cell-by-cell values: plain output");
-    if constexpr (sizeof(T) == 8) {
-      double2* oq = reinterpret_cast<double2*>(out) + e * 2;
-      oq[0] = make_double2(acc[0], acc[1]);
-      oq[1] = make_double2(acc[2], acc[3]);
-    } else {
-      reinterpret_cast<float4*>(out)[e] = make_float4(acc[0], acc[1], acc[2], acc[3]);
-    }
-  } else {
-#pragma unroll
-    for (int i = 0; i < Np; ++i) store_out(out, (int64_t)i * stride + e, acc[i], uu[i]);
-  }
 #pragma unroll
   for (int i = 0; i < Np; ++i) dotv += (double)uu[i] * (double)acc[i];
   return dotv;
 }
 
+template <int DIM, typename T, int VAR, bool PACK = false, class Out = T*, class Slip = NoSlip,
+          class Nodes = TabNodes, bool KAOS = false, bool VCM = false>
+__device__ __forceinline__ double
+apply_p1_cell(int64_t e, int64_t stride, const T* __restrict__ u, const double* __restrict__ Kt,
+              const double* __restrict__ tauS, const int* __restrict__ nbr,
+              const int* __restrict__ code, const int* __restrict__ bctype,
+              const T* __restrict__ kfac, cptr<T> __restrict__ C, cptr<int> __restrict__ tab,
+              Out out, const Slip& slip = Slip{}, const Nodes& nodes = Nodes{}) {
+  constexpr int Np = op_layout(DIM, 1).Np;
+  (void)C;
+  P1Loads<DIM, T> P;
+  p1_load<DIM, T, VAR, PACK, Nodes, KAOS, VCM>(e, stride, u, Kt, tauS, nbr, code, bctype, kfac, tab,
+                                               nodes, P);
+  T acc[Np];
+  const double dotv = p1_compute<DIM, T, VAR>(e, stride, P, slip, acc);
+  if constexpr (VCM) {
+    static_assert(std::is_same<Out, T*>::value, "cell-by-cell values: plain output");
+    p1_store<Np, true>(out, stride, e, acc);
+  } else {
+#pragma unroll
+    for (int i = 0; i < Np; ++i) store_out(out, (int64_t)i * stride + e, acc[i], P.uu[i]);
+  }
+  return dotv;
+}
 
 }  // namespace insp

@@ -6,6 +6,7 @@
 #include <cmath>
 #include <cstring>
 
+#include "cg_kernels.h"
 #include "split_passes.h"
 
 namespace insp {
@@ -14,7 +15,7 @@ namespace {
 // Device scalar slots.
 enum : int {
   S_RZ = 0, S_PAP = 1, S_RR = 2, S_RZN = 3, S_BNUM = 4,
-  S_CG_A = 8, S_CG_PAP = 9, S_CG_B = 10, S_CG_ASAVE = 11,
+  S_CG_A = 8, S_CG_PAP = 9, S_CG_B = 10, S_CG_ASAVE = 11, S_CG_SUM = 15,
   S_EIG_TOP = 12, S_EIG_BOT = 13, S_EIG_NRM = 14,
   S_MEAN = 16, S_BB = 17,
   S_COUNT = 32
@@ -151,7 +152,8 @@ PoissonSolver::PoissonSolver(HostMesh mesh, int order, hipStream_t stream)
   std::vector<int> bt((size_t)std::max<int64_t>(mesh_.n_bfaces, 1), 0);
   bctype_.upload(bt.data(), bt.size());
   scal_.alloc(S_COUNT);
-  partial_.alloc((size_t)std::max<int64_t>(4 * kRedBlocks, split_blocks(E)));
+  // two halves: the coarse CG leaves two sums as partials at a time
+  partial_.alloc((size_t)2 * std::max<int64_t>(4 * kRedBlocks, split_blocks(E)));
   INSP_HIP(hipHostMalloc((void**)&host_scal_, S_COUNT * sizeof(double), hipHostMallocDefault));
 }
 
@@ -905,37 +907,72 @@ void PoissonSolver::coarse_cg(int l) {
     bb = w.ax.p;
     inv = w.d.p;
   }
-  fill<T>(n, w.x.p, (T)0, stream_);
-  jacobi<T>(n, bb, inv, w.z.p, stream_);
-  copy<T>(n, w.z.p, w.p.p, stream_);
-  dot<T>(n, bb, w.z.p, nullptr, nullptr, 1, scal_.p, S_CG_A, rs, stream_);
-  int a = S_CG_A, b = S_CG_B;
+  // The sums are left as partials that the next kernel's blocks add for themselves, or, where there
+  // are too many for that, as one value added up by a kernel in between.
+  double* const part_pap = partial_.p;
+  double* const part_rz = partial_.p + partial_.n / 2;
+  auto folded = [&](int np, double* part, int slot) {
+    if (np <= kFoldParts) return Parts{part, np};
+    finalize(np, 1, part, scal_.p, slot, stream_);
+    return Parts{scal_.p + slot, 1};
+  };
+  const MeshView mv = mesh_view();
+  const LevelView v = level_view(l, std::is_same<T, float>::value);
+  const T* k = var_factor_ ? w.k.p : nullptr;
+  const bool mfma = std::is_same<T, float>::value && matrix_pass(l) && !(oi_ && l == 0);
+  // the apply forms the direction itself on small meshes
+  const bool direction = lv.N == 1 && !has_mass_term() && !(oi_ && l == 0) && !mfma &&
+                         p1_direction_pays(mv);
+  CgSlots c{scal_.p, S_CG_A, S_CG_B, S_CG_PAP, S_CG_ASAVE};
+  const int n0 = cg_init<T>(n, bb, inv, w.x.p, w.z.p, w.p.p, part_rz, stream_);
+  finalize(n0, 1, part_rz, scal_.p, c.rz_old, stream_);
   T* pc = w.p.p;   // the current direction
   T* pq = w.p2.p;  // the previous one (odd iterations) or the buffer for the next one
+  Parts rz{nullptr, 0};
   for (int it = 0; it < pmg_.coarse_iters; ++it) {
-    if (std::is_same<T, float>::value && matrix_pass(l) && !(oi_ && l == 0)) {
+    Parts pap{nullptr, 0};
+    if (it > 0 && direction) {
+      const bool prof = profiling_ && l > 0 && (coarse_sample_++ & 3) == 0;
+      hipEvent_t e0 = nullptr, e1 = nullptr;
+      if (prof) {
+        e0 = ev_take(); e1 = ev_take();
+        INSP_HIP(hipEventRecord(e0, stream_));
+      }
+      launch_p1_direction<T>(mv, v, cells, w.z.p, pc, pq, w.Ap.p, w.x.p, it % 2 == 0, k, rz, c, part_pap,
+                             stream_);
+      if (prof) {
+        INSP_HIP(hipEventRecord(e1, stream_));
+        ev_coarse_.push_back({e0, e1});
+      }
+      std::swap(pc, pq);
+      std::swap(c.rz_old, c.rz_new);
+      pap = folded(apply_blocks(mesh_.n_cells), part_pap, S_CG_SUM);
+    } else if (mfma) {
       // the matrix-core element pass has no fused dot
       apply_level<T>(l, pc, w.Ap.p);
-      dot<T>(n, pc, w.Ap.p, nullptr, nullptr, 1, scal_.p, S_CG_PAP, rs, stream_);
+      dot<T>(n, pc, w.Ap.p, nullptr, nullptr, 1, scal_.p, S_CG_SUM, rs, stream_);
+      pap = Parts{scal_.p + S_CG_SUM, 1};
     } else {
-      const int nparts = apply_level<T>(l, pc, w.Ap.p, partial_.p, nullptr, cells);  // p.Ap fused into the pass
-      finalize(nparts, 1, partial_.p, scal_.p, S_CG_PAP, stream_);
+      const int np = apply_level<T>(l, pc, w.Ap.p, part_pap, nullptr, cells);  // p.Ap fused into the pass
+      pap = folded(np, part_pap, S_CG_SUM);
     }
     ++smoother_applies_;
-    cg_update_z<T>(n, w.z.p, w.Ap.p, inv, scal_.p, a, S_CG_PAP, b, rs, stream_);
+    const int nz = cg_update_z<T>(n, w.z.p, w.Ap.p, inv, pap, c, part_rz, stream_);
     const bool last = it + 1 == pmg_.coarse_iters;
-    if (it % 2 == 1) {
+    if (!last) rz = folded(nz, part_rz, S_CG_SUM);
+    if (last && it % 2 == 0) {
+      cg_update_x<T>(n, w.x.p, pc, c, stream_);
+    } else if (last || (!direction && it % 2 == 1)) {
       // x += alpha_{k-1} p_{k-1} + alpha_k p_k; the next direction overwrites p_{k-1}
-      cg_update_x2p<T>(n, w.x.p, pq, pc, w.z.p, scal_.p, S_CG_ASAVE, a, S_CG_PAP, b, last, stream_);
-      std::swap(pc, pq);
-    } else if (last) {
-      cg_update_xp<T>(n, w.x.p, pc, w.z.p, scal_.p, a, S_CG_PAP, b, true, stream_);
-    } else {
+      cg_update_x2p<T>(n, w.x.p, pq, pc, w.z.p, rz, c, last, stream_);
+    } else if (!direction) {
       // the next direction into the other buffer; alpha_k kept for the x update
-      cg_update_p<T>(n, pq, pc, w.z.p, scal_.p, a, S_CG_PAP, b, S_CG_ASAVE, stream_);
-      std::swap(pc, pq);
+      cg_update_p<T>(n, pq, pc, w.z.p, rz, c, stream_);
     }
-    std::swap(a, b);
+    if (!direction) {
+      std::swap(pc, pq);
+      std::swap(c.rz_old, c.rz_new);
+    }
   }
   if (cells) {
     // x back to rows through ax, then x and ax trade places

@@ -183,136 +183,6 @@ k_cg_update_p(int64_t n, T* __restrict__ p, const T* __restrict__ z, const doubl
     p[i] = fma(beta, p[i], z[i]);
 }
 
-// Jacobi-CG carried in z = D^-1 r (r is never stored): z -= alpha D^-1 Ap, and r.z = sum z^2 / D^-1
-// over the cells (padding entries hold D^-1 = 0 and z = 0).
-template <typename T>
-__global__ void __launch_bounds__(kBlock)
-k_cg_update_z(int64_t n, T* __restrict__ z, const T* __restrict__ Ap, const T* __restrict__ invdiag,
-              const double* __restrict__ scal, int num, int den, double* __restrict__ partial) {
-  const T a = (T)safe_div(scal[num], scal[den]);
-  double v[1] = {0.0};
-  for (int64_t i = blockIdx.x * (int64_t)kBlock + threadIdx.x; i < n; i += (int64_t)gridDim.x * kBlock) {
-    const T di = invdiag[i];
-    const T zi = fma(-a * di, Ap[i], z[i]);
-    z[i] = zi;
-    const double zd = (double)zi;
-    v[0] += di != (T)0 ? zd * zd / (double)di : 0.0;
-  }
-  write_partials<1>(v, partial);
-}
-
-// alpha = scal[anum]/scal[aden], beta = scal[bnum]/scal[anum]: x += alpha p, then p = z + beta p
-// (p is left as it is when last is set).
-template <typename T>
-__global__ void __launch_bounds__(kBlock)
-k_cg_update_xp(int64_t n, T* __restrict__ x, T* __restrict__ p, const T* __restrict__ z,
-               const double* __restrict__ scal, int anum, int aden, int bnum, bool last) {
-  const T a = (T)safe_div(scal[anum], scal[aden]);
-  const T beta = (T)safe_div(scal[bnum], scal[anum]);
-  for (int64_t i = blockIdx.x * (int64_t)kBlock + threadIdx.x; i < n; i += (int64_t)gridDim.x * kBlock) {
-    const T pi = p[i];
-    x[i] = fma(a, pi, x[i]);
-    if (!last) p[i] = fma(beta, pi, z[i]);
-  }
-}
-
-template <typename T>
-__global__ void __launch_bounds__(kBlock)
-k_cg_update_p(int64_t n, T* __restrict__ p_next, const T* __restrict__ p, const T* __restrict__ z,
-              double* __restrict__ scal, int anum, int aden, int bnum, int asave) {
-  const T beta = (T)safe_div(scal[bnum], scal[anum]);
-  for (int64_t i = blockIdx.x * (int64_t)kBlock + threadIdx.x; i < n; i += (int64_t)gridDim.x * kBlock)
-    p_next[i] = fma(beta, p[i], z[i]);
-  // no block reads scal[asave] in this launch
-  if (blockIdx.x == 0 && threadIdx.x == 0) scal[asave] = safe_div(scal[anum], scal[aden]);
-}
-
-template <typename T>
-__global__ void __launch_bounds__(kBlock)
-k_cg_update_x2p(int64_t n, T* __restrict__ x, T* __restrict__ p0, const T* __restrict__ p1,
-                const T* __restrict__ z, const double* __restrict__ scal, int asave, int anum,
-                int aden, int bnum, bool last) {
-  const T a0 = (T)scal[asave];
-  const T a1 = (T)safe_div(scal[anum], scal[aden]);
-  const T beta = (T)safe_div(scal[bnum], scal[anum]);
-  for (int64_t i = blockIdx.x * (int64_t)kBlock + threadIdx.x; i < n; i += (int64_t)gridDim.x * kBlock) {
-    const T q0 = p0[i], q1 = p1[i];
-    x[i] = fma(a1, q1, fma(a0, q0, x[i]));
-    if (!last) p0[i] = fma(beta, q1, z[i]);
-  }
-}
-
-// Two entries per thread with 16-byte (FP64) or 8-byte (FP32) accesses: the direction updates of
-// the coarse CG, whose vectors are even-length and aligned. Same arithmetic per entry as the
-// one-entry kernels.
-template <typename T> struct Pair2;
-template <> struct Pair2<double> { using type = double2; };
-template <> struct Pair2<float> { using type = float2; };
-
-template <typename T>
-__global__ void __launch_bounds__(kBlock)
-k_cg_update_p_pair(int64_t n2, T* __restrict__ p_next, const T* __restrict__ p, const T* __restrict__ z,
-                   double* __restrict__ scal, int anum, int aden, int bnum, int asave) {
-  using V = typename Pair2<T>::type;
-  const T beta = (T)safe_div(scal[bnum], scal[anum]);
-  const int64_t i = blockIdx.x * (int64_t)kBlock + threadIdx.x;
-  if (i < n2) {
-    const V pi = reinterpret_cast<const V*>(p)[i], zi = reinterpret_cast<const V*>(z)[i];
-    V o;
-    o.x = fma(beta, pi.x, zi.x);
-    o.y = fma(beta, pi.y, zi.y);
-    reinterpret_cast<V*>(p_next)[i] = o;
-  }
-  // no block reads scal[asave] in this launch
-  if (blockIdx.x == 0 && threadIdx.x == 0) scal[asave] = safe_div(scal[anum], scal[aden]);
-}
-
-template <typename T>
-__global__ void __launch_bounds__(kBlock)
-k_cg_update_x2p_pair(int64_t n2, T* __restrict__ x, T* __restrict__ p0, const T* __restrict__ p1,
-                     const T* __restrict__ z, const double* __restrict__ scal, int asave, int anum,
-                     int aden, int bnum, bool last) {
-  using V = typename Pair2<T>::type;
-  const T a0 = (T)scal[asave];
-  const T a1 = (T)safe_div(scal[anum], scal[aden]);
-  const T beta = (T)safe_div(scal[bnum], scal[anum]);
-  const int64_t i = blockIdx.x * (int64_t)kBlock + threadIdx.x;
-  if (i >= n2) return;
-  const V q0 = reinterpret_cast<const V*>(p0)[i], q1 = reinterpret_cast<const V*>(p1)[i];
-  V xi = reinterpret_cast<V*>(x)[i];
-  xi.x = fma(a1, q1.x, fma(a0, q0.x, xi.x));
-  xi.y = fma(a1, q1.y, fma(a0, q0.y, xi.y));
-  reinterpret_cast<V*>(x)[i] = xi;
-  if (!last) {
-    const V zi = reinterpret_cast<const V*>(z)[i];
-    V o;
-    o.x = fma(beta, q1.x, zi.x);
-    o.y = fma(beta, q1.y, zi.y);
-    reinterpret_cast<V*>(p0)[i] = o;
-  }
-}
-
-template <typename T>
-__global__ void __launch_bounds__(kBlock)
-k_cg_update_z_pair(int64_t n2, T* __restrict__ z, const T* __restrict__ Ap,
-                   const T* __restrict__ invdiag, const double* __restrict__ scal, int num, int den,
-                   double* __restrict__ partial) {
-  using V = typename Pair2<T>::type;
-  const T a = (T)safe_div(scal[num], scal[den]);
-  double v[1] = {0.0};
-  for (int64_t i = blockIdx.x * (int64_t)kBlock + threadIdx.x; i < n2; i += (int64_t)gridDim.x * kBlock) {
-    const V di = reinterpret_cast<const V*>(invdiag)[i], api = reinterpret_cast<const V*>(Ap)[i];
-    V zi = reinterpret_cast<V*>(z)[i];
-    zi.x = fma(-a * di.x, api.x, zi.x);
-    zi.y = fma(-a * di.y, api.y, zi.y);
-    reinterpret_cast<V*>(z)[i] = zi;
-    const double zx = (double)zi.x, zy = (double)zi.y;
-    v[0] += di.x != (T)0 ? zx * zx / (double)di.x : 0.0;
-    v[0] += di.y != (T)0 ? zy * zy / (double)di.y : 0.0;
-  }
-  write_partials<1>(v, partial);
-}
-
 template <typename T>
 __global__ void __launch_bounds__(kBlock)
 k_jacobi(int64_t n, const T* __restrict__ r, const T* __restrict__ invdiag, T* __restrict__ z) {
@@ -553,15 +423,6 @@ __global__ void k_scal_copy(double* scal, int dst, int src) {
   if (threadIdx.x == 0) scal[dst] = scal[src];
 }
 
-// Vectors that the pair kernels may take: an even length and every base aligned to two entries.
-template <typename T>
-bool pairs_ok(int64_t n, std::initializer_list<const void*> ptrs) {
-  if (n & 1) return false;
-  for (const void* q : ptrs)
-    if (reinterpret_cast<uintptr_t>(q) % (2 * sizeof(T)) != 0) return false;
-  return true;
-}
-
 // Vectors that the 16-byte kernels may take: a length that is a multiple of the entries per
 // access and every base (null ones aside) 16-byte aligned.
 template <typename T>
@@ -651,52 +512,6 @@ template <typename T>
 void cg_update_p(int64_t n, T* p, const T* z, const double* scal, int num, int den, hipStream_t s) {
   hipLaunchKernelGGL((k_cg_update_p<T>), dim3(grid_stream(n)), dim3(kBlock), 0, s, n, p, z, scal,
                      num, den); launch_check("k_cg_update_p");
-}
-
-template <typename T>
-void cg_update_z(int64_t n, T* z, const T* Ap, const T* invdiag, double* scal, int num, int den,
-                 int out, RedScratch rs, hipStream_t s) {
-  const int nb = red_blocks(n);
-  if (pairs_ok<T>(n, {z, Ap, invdiag})) {
-    hipLaunchKernelGGL((k_cg_update_z_pair<T>), dim3(nb), dim3(kBlock), 0, s, n / 2, z, Ap, invdiag,
-                       scal, num, den, rs.partial); launch_check("k_cg_update_z_pair");
-  } else {
-    hipLaunchKernelGGL((k_cg_update_z<T>), dim3(nb), dim3(kBlock), 0, s, n, z, Ap, invdiag, scal, num,
-                       den, rs.partial); launch_check("k_cg_update_z");
-  }
-  hipLaunchKernelGGL(k_finalize, dim3(1), dim3(kFinBlock), 0, s, nb, 1, rs.partial, scal, out); launch_check("k_finalize");
-}
-
-template <typename T>
-void cg_update_xp(int64_t n, T* x, T* p, const T* z, const double* scal, int anum, int aden,
-                  int bnum, bool last, hipStream_t s) {
-  hipLaunchKernelGGL((k_cg_update_xp<T>), dim3(grid_stream(n)), dim3(kBlock), 0, s, n, x, p, z, scal,
-                     anum, aden, bnum, last); launch_check("k_cg_update_xp");
-}
-
-template <typename T>
-void cg_update_p(int64_t n, T* p_next, const T* p, const T* z, double* scal, int anum, int aden,
-                 int bnum, int asave, hipStream_t s) {
-  if (pairs_ok<T>(n, {p_next, p, z})) {
-    hipLaunchKernelGGL((k_cg_update_p_pair<T>), dim3(grid_stream(n / 2)), dim3(kBlock), 0, s, n / 2,
-                       p_next, p, z, scal, anum, aden, bnum, asave); launch_check("k_cg_update_p_pair");
-    return;
-  }
-  hipLaunchKernelGGL((k_cg_update_p<T>), dim3(grid_stream(n)), dim3(kBlock), 0, s, n, p_next, p, z, scal,
-                     anum, aden, bnum, asave); launch_check("k_cg_update_p");
-}
-
-template <typename T>
-void cg_update_x2p(int64_t n, T* x, T* p0, const T* p1, const T* z, const double* scal, int asave,
-                   int anum, int aden, int bnum, bool last, hipStream_t s) {
-  if (pairs_ok<T>(n, {x, p0, p1, z})) {
-    hipLaunchKernelGGL((k_cg_update_x2p_pair<T>), dim3(grid_stream(n / 2)), dim3(kBlock), 0, s, n / 2,
-                       x, p0, p1, z, scal, asave, anum, aden, bnum, last);
-    launch_check("k_cg_update_x2p_pair");
-    return;
-  }
-  hipLaunchKernelGGL((k_cg_update_x2p<T>), dim3(grid_stream(n)), dim3(kBlock), 0, s, n, x, p0, p1, z,
-                     scal, asave, anum, aden, bnum, last); launch_check("k_cg_update_x2p");
 }
 
 template <typename T>
@@ -834,14 +649,6 @@ void scal_copy(double* scal, int dst, int src, hipStream_t s) {
   template void cg_update_xr<T>(int64_t, T*, T*, const T*, const T*, const T*, T*, double*, int,  \
                                 int, int, RedScratch, hipStream_t);                               \
   template void cg_update_p<T>(int64_t, T*, const T*, const double*, int, int, hipStream_t);      \
-  template void cg_update_z<T>(int64_t, T*, const T*, const T*, double*, int, int, int,           \
-                               RedScratch, hipStream_t);                                          \
-  template void cg_update_xp<T>(int64_t, T*, T*, const T*, const double*, int, int, int, bool,    \
-                                hipStream_t);                                                     \
-  template void cg_update_p<T>(int64_t, T*, const T*, const T*, double*, int, int, int, int,      \
-                               hipStream_t);                                                      \
-  template void cg_update_x2p<T>(int64_t, T*, T*, const T*, const T*, const double*, int, int,    \
-                                 int, int, bool, hipStream_t);                                    \
   template void jacobi<T>(int64_t, const T*, const T*, T*, hipStream_t);                          \
   template void cheb_step<T>(int64_t, const T*, const T*, const T*, T*, T*, T, T, bool,           \
                              hipStream_t);                                                        \

@@ -46,3 +46,52 @@ def test_apply_both_forms(ip, oracle, dim, N, n, factor):
     y = o.mult(x)
     assert rel(s.mult(x), y) < (1e-12 if N < 4 else 1e-11)
     assert rel(s.mult_fp32(x), y) < 2e-5
+
+
+@pytest.mark.parametrize("dim,n", [(2, 250), (3, 28)])
+@pytest.mark.parametrize("factor", [False, True])
+def test_order1_apply_repeats(ip, oracle, dim, n, factor):
+    """Several waves per SIMD: every launch of the order-1 pass gives the same bits, and the oracle's
+    values (1e-12: at most 40 terms per entry)."""
+    mesh = ip.Mesh.square(n, jitter=0.1, seed=5) if dim == 2 else ip.Mesh.cube(n, 0.1, 5)
+    s = ip.PoissonSolver(mesh, 1)
+    o = oracle.Oracle(*mesh.arrays(), 1)
+    s.set_solver(ip.SOLVER_JACOBI)
+    rng = np.random.default_rng(n)
+    if factor:
+        k = 1.0 + rng.random((s.n_cells, s.Np))
+        s.set_factor(k)
+        o.set_factor(k)
+    x = rng.standard_normal((s.n_cells, s.Np))
+    y = s.mult(x)
+    assert rel(y, o.mult(x)) < 1e-12
+    for _ in range(20):
+        assert np.array_equal(s.mult(x), y)
+
+
+@pytest.mark.parametrize("dim,n,iters", [(2, 4, 1), (2, 4, 2), (2, 30, 7), (3, 3, 8), (3, 12, 9), (3, 27, 12),
+                                         (3, 33, 12)])
+@pytest.mark.parametrize("mixed", [False, True])
+@pytest.mark.parametrize("factor", [False, True])
+def test_coarse_cg_forms(ip, oracle, dim, n, iters, mixed, factor):
+    """The order-1 Jacobi-CG with the direction formed in the apply (small meshes), as updates of their
+    own, with sums folded into the next kernel and added by a kernel in between; odd and even counts.
+    The preconditioned solve must end at the oracle's residual and take the same iterations twice."""
+    mesh = ip.Mesh.square(n, jitter=0.1, seed=5) if dim == 2 else ip.Mesh.cube(n, 0.1, 5)
+    s = ip.PoissonSolver(mesh, 2)
+    o = oracle.Oracle(*mesh.arrays(), 2)
+    rng = np.random.default_rng(n)
+    if factor:
+        k = 1.0 + rng.random((s.n_cells, s.Np))
+        s.set_factor(k)
+        o.set_factor(k)
+    s.set_pmg([2, 1], coarse_iters=iters)
+    s.set_precision(ip.PRECISION_MIXED if mixed else ip.PRECISION_FP64)
+    s.set_tol_and_iter(1e-9, 0.0, 2000)
+    b = rng.standard_normal((s.n_cells, s.Np))
+    x, y = np.zeros_like(b), np.zeros_like(b)
+    assert s.solve(b, x)
+    its = s.last_stats["iterations"]
+    assert np.linalg.norm(b - o.mult(x)) <= 2e-9 * np.linalg.norm(b)
+    assert s.solve(b, y) and s.last_stats["iterations"] == its
+    assert np.array_equal(x, y)
