@@ -22,7 +22,8 @@ SOURCES = ["refelem.cpp", "mesh.cpp", "hdf5_reader.cpp", "solver.cpp", "viscous_
            "amg_kernels.hip", "block_kernels.hip", "rhs_kernels.hip", "sipg_mfma.hip",
            "probe_kernels.hip", "mass_kernels.hip",
            "proj_kernels.hip", "sipg_oi.hip", "sipg_split.hip", "cg_kernels.hip",
-           "sipg_split_3d3.hip", "sipg_split_3d4.hip", "sipg_split_3d4f.hip"]
+           "sipg_split_3d3.hip", "sipg_split_3d4.hip", "sipg_split_3d4f.hip",
+           "sipg_split_vec.hip", "sipg_split_vec3d4.hip", "sipg_mass.hip", "pcg_kernels.hip"]
 
 COMMON = ["-O3", "-std=c++17", "-fPIC", f"--offload-arch={ARCH}",
           # packed FP32 instructions are disabled for all device code

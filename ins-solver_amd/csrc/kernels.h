@@ -57,6 +57,14 @@ struct LevelView {
   const double* tau_cells = nullptr;  // [E][4] tauS cell by cell (3D order 1), or null
 };
 
+// The mass term of the viscous operator (J M (mm o u), or mmc J M u) for an element pass to add.
+template <typename T>
+struct MassView {
+  const T* mm = nullptr;  // per-node factor, or null
+  T mmc = 0;              // constant factor
+  bool on() const { return mm != nullptr || mmc != (T)0; }
+};
+
 // SIPG operator: trace pass + element pass (order 1: element pass only). With
 // `partial` the element pass also writes per-block partial sums of u.(A u)
 // (apply_blocks(E) of them) for a deterministic finalize.
@@ -66,6 +74,10 @@ void launch_trace(const MeshView& m, const LevelView& l, const T* u, const T* kf
 template <typename T>
 void launch_apply(const MeshView& m, const LevelView& l, const T* u, const T* tr, const T* kfac,
                   T* out, hipStream_t s, double* partial = nullptr);
+// The same with the mass term added by the element pass (orders >= 2, packed words, FP64).
+void launch_apply_mass(const MeshView& m, const LevelView& l, const double* u, const double* tr,
+                       const double* kfac, const MassView<double>& mass, double* out, hipStream_t s,
+                       double* partial);
 int apply_blocks(int64_t E);
 // Order-1 apply (3D, with the cell-by-cell metric) on values held cell by cell: u and out are
 // [E][4] (the coarse Jacobi-CG runs on such copies); the coefficient stays in rows.

@@ -41,6 +41,40 @@ __device__ __forceinline__ T kval(const T* __restrict__ kfac, int64_t idx) {
   else return kfac ? kfac[idx] : (T)1;
 }
 
+// Mass term of the viscous operator, J M (mm o u) (per node from mm, else the constant mmc), where on.
+template <typename T>
+struct MassTerm {
+  const double* J = nullptr;
+  const T* mm = nullptr;
+  T mmc = 0;
+  bool on = false;
+};
+
+// Its node columns one after the other, in the volume term's loop over them. The column's value is
+// loaded again (registers have no run-time index) one column ahead, so that its wait lies behind a
+// column's arithmetic; the unrolled form keeps all of M in spilled scalar registers.
+template <typename T>
+struct MassColumns {
+  const MassTerm<T>& m;
+  const T* __restrict__ u;
+  int64_t e, stride;
+  T Je, next;
+  __device__ __forceinline__ T load(int j) const {
+    return (m.mm ? m.mm[j * stride + e] : m.mmc) * u[j * stride + e];
+  }
+  __device__ __forceinline__ MassColumns(const MassTerm<T>& mass, const T* __restrict__ uu, int64_t cell,
+                                         int64_t st, int j0, bool on)
+      : m(mass), u(uu), e(cell), stride(st), Je(on ? (T)mass.J[cell] : (T)0), next(on ? load(j0) : (T)0) {}
+  // acc += column j; j1: the end of the loop
+  template <int Np>
+  __device__ __forceinline__ void add(int j, int j1, cptr<T> __restrict__ row, T (&acc)[Np]) {
+    const T v = Je * next;
+    next = load(j + 1 < j1 ? j + 1 : j);
+#pragma unroll
+    for (int i = 0; i < Np; ++i) acc[i] = fma(row[i], v, acc[i]);
+  }
+};
+
 // Trace pass for one cell: T = sJ n.(k grad u) at every face node. Per node h = k K grad u is
 // formed once; a face's trace is sum_r alpha_{f,r} h_r with the compile-time face coefficients
 // (one row of h, or the sum of its rows on the slanted face), so no per-face coefficient table
@@ -135,13 +169,14 @@ constexpr int face_chunk(int dim, int N, int bytes) {
 // One cell of the element pass; returns u.(A u) over the cell. PACK: nbr holds the packed
 // words (neighbour << 5) | code, -(bface+1) on the boundary, and code is not read.
 template <int DIM, int N, typename T, int VAR, bool PACK = false, class Out = T*,
-          class Slip = NoSlip>
+          class Slip = NoSlip, bool MASS = false>
 __device__ __forceinline__ double
 apply_cell(int64_t e, int64_t stride, const T* __restrict__ u, const T* __restrict__ tr,
            const double* __restrict__ Kt, const double* __restrict__ tauS,
            const int* __restrict__ nbr, const int* __restrict__ code,
            const int* __restrict__ bctype, const T* __restrict__ kfac, cptr<T> __restrict__ C,
-           cptr<int> __restrict__ tab, Out out, const Slip& slip = Slip{}) {
+           cptr<int> __restrict__ tab, Out out, const Slip& slip = Slip{},
+           const MassTerm<T>& mass = MassTerm<T>{}) {
   constexpr OpLayout L = op_layout(DIM, N);
   constexpr int Np = L.Np, Nfp = L.Nfp, Nf = L.Nf;
   constexpr FmaskTable FM = make_fmask(DIM, N);
@@ -170,6 +205,7 @@ apply_cell(int64_t e, int64_t stride, const T* __restrict__ u, const T* __restri
   }
 
   // Volume term, one node column at a time.
+  MassColumns<T> mc(mass, u, e, stride, 0, MASS);
   for (int j = 0; j < Np; ++j) {
     T g[DIM];
 #pragma unroll
@@ -190,6 +226,7 @@ apply_cell(int64_t e, int64_t stride, const T* __restrict__ u, const T* __restri
 #pragma unroll
       for (int i = 0; i < Np; ++i) acc[i] = fma(C[L.off_Bt + (r * Np + j) * Np + i], h, acc[i]);
     }
+    if constexpr (MASS) mc.add(j, Np, C + L.off_M + j * Np, acc);
   }
 
   // Face terms. The face nodes are taken in chunks of CH; the loads of a chunk are issued in

@@ -81,16 +81,7 @@ trace_quarter(int64_t e, int64_t stride, const T (&uu)[op_layout(DIM, N).Np],
   }
 }
 
-// Volume term of the node columns [j0, j1), with the mass term J M (mm o u) of those columns when
-// mm_on (per node from mm, else the constant mmc).
-template <typename T>
-struct MassTerm {
-  const double* J = nullptr;
-  const T* mm = nullptr;
-  T mmc = 0;
-  bool on = false;
-};
-
+// Volume term of the node columns [j0, j1), and their mass term.
 template <int DIM, int N, typename T, int VAR>
 __device__ __forceinline__ void
 volume_columns(int64_t e, int64_t stride, int j0, int j1, const T (&uu)[op_layout(DIM, N).Np],
@@ -98,7 +89,7 @@ volume_columns(int64_t e, int64_t stride, int j0, int j1, const T (&uu)[op_layou
                cptr<T> __restrict__ C, const MassTerm<T>& mass, T (&acc)[op_layout(DIM, N).Np]) {
   constexpr OpLayout L = op_layout(DIM, N);
   constexpr int Np = L.Np;
-  const T Je = mass.on ? (T)mass.J[e] : (T)0;
+  MassColumns<T> mc(mass, u, e, stride, j0, mass.on);
 #pragma unroll 1
   for (int j = j0; j < j1; ++j) {
     T g[DIM];
@@ -119,11 +110,7 @@ volume_columns(int64_t e, int64_t stride, int j0, int j1, const T (&uu)[op_layou
 #pragma unroll
       for (int i = 0; i < Np; ++i) acc[i] = fma(C[L.off_Bt + (r * Np + j) * Np + i], h, acc[i]);
     }
-    if (mass.on) {
-      const T v = Je * (mass.mm ? mass.mm[j * stride + e] : mass.mmc) * u[j * stride + e];
-#pragma unroll
-      for (int i = 0; i < Np; ++i) acc[i] = fma(C[L.off_M + j * Np + i], v, acc[i]);
-    }
+    if (mass.on) mc.add(j, j1, C + L.off_M + j * Np, acc);
   }
 }
 
@@ -141,6 +128,7 @@ apply_quarter(int64_t e, int64_t stride, const T* __restrict__ u, const T* __res
   constexpr int Np = L.Np, Nfp = L.Nfp, Nf = L.Nf;
   constexpr FmaskTable FM = make_fmask(DIM, N);
   constexpr SplitCols<DIM, N> cols;
+  static_assert(cols.b[W] < cols.b[W + 1], "every wave has a column");
   constexpr bool has_face = W < Nf;
   constexpr int F0 = has_face ? W : 0;
   int nb = 0;

@@ -10,6 +10,12 @@ INSP_SPLIT_INST(extern, 3, 3, double)
 INSP_SPLIT_INST(extern, 3, 3, float)
 INSP_SPLIT_INST(extern, 3, 4, double)
 INSP_SPLIT_INST(extern, 3, 4, float)
+INSP_SPLIT_VEC(extern, 2, 2)
+INSP_SPLIT_VEC(extern, 2, 3)
+INSP_SPLIT_VEC(extern, 2, 4)
+INSP_SPLIT_VEC(extern, 3, 2)
+INSP_SPLIT_VEC(extern, 3, 3)
+INSP_SPLIT_VEC(extern, 3, 4)
 }  // namespace split
 
 namespace {
@@ -47,9 +53,9 @@ int split_blocks(int64_t E) { return (int)split::grid_split(E).x; }
 
 template <typename T>
 void launch_trace_split(const MeshView& m, const LevelView& l, const T* u, const T* kfac, T* tr,
-                        hipStream_t s) {
+                        hipStream_t s, int ncomp, int64_t cs, int64_t ts) {
   if (m.E == 0) return;
-  INSP_SPLIT_N(m.dim, l.N, (split::trace<D_, N_, T>(m, l, u, kfac, tr, s)))
+  INSP_SPLIT_N(m.dim, l.N, (split::trace<D_, N_, T>(m, l, u, kfac, tr, s, ncomp, cs, ts)))
 }
 
 template <typename T>
@@ -66,9 +72,16 @@ void launch_cheb_split(const MeshView& m, const LevelView& l, const T* u, const 
   INSP_SPLIT_N(m.dim, l.N, (split::cheb<D_, N_, T>(m, l, u, tr, kfac, f, inv, prev, x_next, c1, c2, s)))
 }
 
+void launch_vec_split(const MeshView& m, const LevelView& l, int ncomp, const double* u, const double* tr,
+                      const double* kfac, const MassView<double>& mass, const double* bnormal, int64_t cs,
+                      int64_t ts, int64_t bs, double* out, hipStream_t s, double* partial) {
+  if (m.E == 0) return;
+  INSP_SPLIT_N(m.dim, l.N, (split::vec<D_, N_>(m, l, ncomp, u, tr, kfac, mass, bnormal, cs, ts, bs, out, s, partial)))
+}
+
 #define INSP_INST(T)                                                                                   \
   template void launch_trace_split<T>(const MeshView&, const LevelView&, const T*, const T*, T*,       \
-                                      hipStream_t);                                                    \
+                                      hipStream_t, int, int64_t, int64_t);                                                    \
   template void launch_apply_split<T>(const MeshView&, const LevelView&, const T*, const T*, const T*, \
                                       const MassView<T>&, T*, hipStream_t, double*);                   \
   template void launch_cheb_split<T>(const MeshView&, const LevelView&, const T*, const T*, const T*,  \

@@ -7,6 +7,7 @@
 #include <cstring>
 
 #include "cg_kernels.h"
+#include "pcg_kernels.h"
 #include "split_passes.h"
 
 namespace insp {
@@ -151,10 +152,11 @@ PoissonSolver::PoissonSolver(HostMesh mesh, int order, hipStream_t stream)
   }
   std::vector<int> bt((size_t)std::max<int64_t>(mesh_.n_bfaces, 1), 0);
   bctype_.upload(bt.data(), bt.size());
-  scal_.alloc(S_COUNT);
+  scal_.alloc(S_COUNT + P_COUNT);
   // two halves: the coarse CG leaves two sums as partials at a time
   partial_.alloc((size_t)2 * std::max<int64_t>(4 * kRedBlocks, split_blocks(E)));
-  INSP_HIP(hipHostMalloc((void**)&host_scal_, S_COUNT * sizeof(double), hipHostMallocDefault));
+  INSP_HIP(hipHostMalloc((void**)&host_scal_, (S_COUNT + 2 * P_COUNT) * sizeof(double), hipHostMallocDefault));
+  for (hipEvent_t& e : ev_pcg_) INSP_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
 }
 
 PoissonSolver::~PoissonSolver() {
@@ -165,6 +167,8 @@ PoissonSolver::~PoissonSolver() {
   std::sort(ev_pool_.begin(), ev_pool_.end());
   ev_pool_.erase(std::unique(ev_pool_.begin(), ev_pool_.end()), ev_pool_.end());
   for (auto ev : ev_pool_) (void)hipEventDestroy(ev);
+  for (hipEvent_t e : ev_pcg_)
+    if (e) (void)hipEventDestroy(e);
   if (host_scal_) (void)hipHostFree(host_scal_);
   if (own_stream_) (void)hipStreamDestroy(stream_);
 }
@@ -759,7 +763,14 @@ int PoissonSolver::apply_level(int l, const T* u, T* out, double* partial, T* tr
   } else {
     trace_pass<T>(mv, v, u, k, tr, stream_);
     if (prof) INSP_HIP(hipEventRecord(e1, stream_));
-    launch_apply<T>(mv, v, u, tr, k, out, stream_, partial);
+    if constexpr (std::is_same<T, double>::value) {
+      if (has_mass_term() && mv.nbc && lv.N >= 2) {
+        launch_apply_mass(mv, v, u, tr, k, MassView<double>{var_mm_ ? w.mm.p : nullptr, mm_const_}, out,
+                          stream_, partial);
+        mass_done = true;
+      }
+    }
+    if (!mass_done) launch_apply<T>(mv, v, u, tr, k, out, stream_, partial);
   }
   if (has_mass_term() && !mass_done) {
     if (cells) throw std::logic_error("cell-by-cell apply with a mass term");
@@ -1417,6 +1428,37 @@ void PoissonSolver::set_dat_stride(int64_t s) {
   dat_stride_ = s;
 }
 
+bool PoissonSolver::fused_pcg() const {
+  return (type_ == SolverType::JACOBI_PCG || type_ == SolverType::INV_MASS_PCG) && !nullspace_;
+}
+
+// At most `limit` iterations of the Jacobi or inverse-mass CG from r_, z_ = p_ and r.z in its first slot;
+// x_ and r_ are those of the last one.
+PcgEnd PoissonSolver::pcg_iterate(double tol, int limit) {
+  const int64_t n = (int64_t)np() * stride_;
+  double* const st = scal_.p + S_COUNT;
+  double* const part_pap = partial_.p;
+  double* const part_step = partial_.p + partial_.n / 2;
+  pcg_start(st, stream_);
+  auto step = [&](int k) {
+    const int rz = P_RZ0 + k % 2, rz_next = P_RZ0 + (k + 1) % 2;
+    Parts pap{part_pap, apply_level<double>(0, p_.p, Ap_.p, part_pap)};  // p.Ap fused into the element pass
+    if (pap.n > kFoldParts) {
+      finalize(pap.n, 1, part_pap, st, P_SUM, stream_);
+      pap = Parts{st + P_SUM, 1};
+    }
+    const int nb = type_ == SolverType::JACOBI_PCG
+                       ? pcg_update_jacobi(n, x_.p, r_.p, z_.p, p_.p, Ap_.p, levels_[0]->w64.inv.p, pap, st, rz,
+                                           part_step, stream_)
+                       : pcg_update_inv_mass(np(), 1, mesh_.n_cells, stride_, 0, x_.p, r_.p, z_.p, p_.p, Ap_.p,
+                                             J_.p, minv_.p, inv_mass_factor_,
+                                             inv_mass_recp_.empty() ? nullptr : inv_mass_recp_.p, pap, st, rz,
+                                             part_step, stream_);
+    pcg_direction(n, p_.p, z_.p, nb, part_step, st, rz, rz_next, tol, stream_);
+  };
+  return pcg_drive(limit, n <= kAheadEntries, st, host_scal_ + S_COUNT, ev_pcg_, stream_, step);
+}
+
 int PoissonSolver::solve(const double* rhs, double* ans, Layout layout, SolveStats* stats) {
   if (!initialised_) init();
   const auto t0 = std::chrono::steady_clock::now();
@@ -1459,8 +1501,15 @@ int PoissonSolver::solve(const double* rhs, double* ans, Layout layout, SolveSta
       if (std::sqrt(rr_true) <= tol) { status = 0; break; }
       if (it >= max_iter_ || restart > 50) { status = 1; break; }
       precondition(r, z_.p);
-      dot<double>(n, r, z_.p, nullptr, nullptr, 1, scal_.p, S_RZ, rs, stream_);
+      dot<double>(n, r, z_.p, nullptr, nullptr, 1, scal_.p, fused_pcg() ? S_COUNT + P_RZ0 : S_RZ, rs, stream_);
       copy<double>(n, z_.p, p_.p, stream_);
+      if (fused_pcg()) {
+        const PcgEnd end = pcg_iterate(tol, max_iter_ - it);
+        it += end.iterations;
+        fine_applies += end.iterations;
+        if (end.stop == PCG_BREAKDOWN) { status = -3; break; }
+        continue;
+      }
       bool breakdown = false;
       while (it < max_iter_) {
         const int nparts = apply_level<double>(0, p_.p, Ap_.p, partial_.p);  // p.Ap fused into the element pass

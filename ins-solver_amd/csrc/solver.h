@@ -18,6 +18,7 @@
 #include "kernels.h"
 #include "mesh.h"
 #include "oi.h"
+#include "pcg_kernels.h"
 #include "refelem.h"
 #include "vec_kernels.h"
 
@@ -253,6 +254,10 @@ class PoissonSolver {
   template <typename T>
   void coarse_amg(int l);
   void precondition(const double* r, double* z);
+  // Jacobi and inverse-mass CG with fused iterations (pcg_kernels.h); the mean projection of a pure
+  // Neumann problem keeps the general loop.
+  bool fused_pcg() const;
+  PcgEnd pcg_iterate(double tol, int limit);
   // FP32 inner iterations with FP64 iterate, true residuals and step lengths (p-multigrid
   // with Precision::MIXED); returns the solve status.
   bool mixed_refinement() const;
@@ -327,6 +332,7 @@ class PoissonSolver {
   DBuf<double> scal_;
   DBuf<double> partial_;
   double* host_scal_ = nullptr;  // pinned
+  hipEvent_t ev_pcg_[2] = {nullptr, nullptr};
   int64_t smoother_applies_ = 0;
 
   bool profiling_ = false;

@@ -23,18 +23,19 @@ namespace insp {
 bool split_trace(const MeshView& m, const LevelView& l);
 bool split_apply(const MeshView& m, const LevelView& l, bool fp32);
 int split_blocks(int64_t E);  // partials of u.(A u) that the split element pass leaves
+// ncomp vectors cs apart, their traces ts apart
 template <typename T>
 void launch_trace_split(const MeshView& m, const LevelView& l, const T* u, const T* kfac, T* tr,
-                        hipStream_t s);
-// The mass term of the viscous operator (J M (mm o u), or mmc J M u), added by the split element pass.
-template <typename T>
-struct MassView {
-  const T* mm = nullptr;  // per-node factor, or null
-  T mmc = 0;              // constant factor
-};
+                        hipStream_t s, int ncomp = 1, int64_t cs = 0, int64_t ts = 0);
 template <typename T>
 void launch_apply_split(const MeshView& m, const LevelView& l, const T* u, const T* tr, const T* kfac,
                         const MassView<T>& mass, T* out, hipStream_t s, double* partial);
+// Every component of the vector (velocity) operator (launch_apply_slip, kernels.h) in one launch:
+// vectors, traces and bc types of the components lie cs, ts and bs apart; split_blocks(E) partials a
+// component.
+void launch_vec_split(const MeshView& m, const LevelView& l, int ncomp, const double* u, const double* tr,
+                      const double* kfac, const MassView<double>& mass, const double* bnormal, int64_t cs,
+                      int64_t ts, int64_t bs, double* out, hipStream_t s, double* partial);
 template <typename T>
 void launch_cheb_split(const MeshView& m, const LevelView& l, const T* u, const T* tr, const T* kfac,
                        const T* f, const T* inv, const T* prev, T* x_next, T c1, T c2, hipStream_t s);

@@ -4,6 +4,7 @@
 #include <cmath>
 
 #include "kernels.h"
+#include "pcg_kernels.h"
 #include "refelem.h"
 #include "split_passes.h"
 #include "vec_kernels.h"
@@ -12,6 +13,7 @@ namespace insp {
 
 namespace {
 enum VecSlot { V_RZ = 0, V_PAP = 1, V_RR = 2, V_RZN = 3, V_BNUM = 4, V_BB = 5, V_COUNT = 8 };
+
 }  // namespace
 
 VecViscousSolver::VecViscousSolver(HostMesh mesh, int order) : base_(std::move(mesh), order) {
@@ -40,8 +42,8 @@ VecViscousSolver::VecViscousSolver(HostMesh mesh, int order) : base_(std::move(m
   bn_.upload(bn.data(), bn.size());
   std::vector<int> eff((size_t)ncomp_ * std::max<int64_t>(B, 1), 0);
   eff_.upload(eff.data(), eff.size());
-  scal_.alloc(V_COUNT);
-  INSP_HIP(hipHostMalloc((void**)&host_scal_, V_COUNT * sizeof(double), hipHostMallocDefault));
+  scal_.alloc(V_COUNT + P_COUNT);
+  INSP_HIP(hipHostMalloc((void**)&host_scal_, (V_COUNT + 2 * P_COUNT) * sizeof(double), hipHostMallocDefault));
 }
 
 VecViscousSolver::~VecViscousSolver() {
@@ -108,7 +110,8 @@ void VecViscousSolver::init() {
   const size_t n = (size_t)ncomp_ * Np * st;
   b_.alloc(n); x_.alloc(n); r_.alloc(n); z_.alloc(n); zold_.alloc(n); p_.alloc(n); Ap_.alloc(n);
   tr_.alloc((size_t)ncomp_ * base_.fine_face_nodes() * st);
-  partial_.alloc((size_t)std::max<int64_t>(4 * kRedBlocks, (int64_t)ncomp_ * apply_blocks(E)));
+  // two halves: the step's sums beside those of the element passes
+  partial_.alloc((size_t)2 * std::max<int64_t>(4 * kRedBlocks, (int64_t)ncomp_ * split_blocks(E)));
   const std::vector<double> Mi = mat_inverse(base_.fine_re_.M, Np);
   minv_.upload(Mi.data(), Mi.size());
   inv_.release();
@@ -139,14 +142,29 @@ void VecViscousSolver::init() {
 }
 
 // Traces of every component (orders >= 2), then the element pass of each component.
-void VecViscousSolver::apply(const double* u, double* out, double* partial) {
+int VecViscousSolver::apply(const double* u, double* out, double* partial) {
   const MeshView mv = base_.mesh_view();
   const LevelView lv = base_.level_view(0, false);
   const double* k = base_.fine_factor();
   const int64_t cs = (int64_t)base_.np() * base_.stride_;
   const int64_t ts = (int64_t)base_.fine_face_nodes() * base_.stride_;
-  for (int c = 0; c < ncomp_; ++c) trace_pass<double>(mv, lv, u + c * cs, k, tr_.p + c * ts, base_.stream_);
+  if (split_trace(mv, lv))
+    launch_trace_split<double>(mv, lv, u, k, tr_.p, base_.stream_, ncomp_, cs, ts);
+  else
+    for (int c = 0; c < ncomp_; ++c) launch_trace<double>(mv, lv, u + c * cs, k, tr_.p + c * ts, base_.stream_);
+  // the components' cells run together
+  MeshView all = mv;
+  all.E *= ncomp_;
+  if (split_apply(all, lv, false)) {
+    const int64_t bs = std::max<int64_t>(base_.mesh_.n_bfaces, 1);
+    MeshView m = mv;
+    m.bctype = eff_.p;
+    launch_vec_split(m, lv, ncomp_, u, tr_.p, k, MassView<double>{base_.fine_mm(), base_.mm_const_}, bn_.p, cs,
+                     ts, bs, out, base_.stream_, partial);
+    return ncomp_ * split_blocks(mv.E);
+  }
   for (int c = 0; c < ncomp_; ++c) apply_one(c, u, out + c * cs, partial);
+  return ncomp_ * apply_blocks(mv.E);
 }
 
 // Component c of A u (the traces of every component already in tr_).
@@ -313,6 +331,38 @@ void VecViscousSolver::apply_bc(double* const rhs[], Layout layout) {
   INSP_HIP(hipStreamSynchronize(base_.stream_));
 }
 
+bool VecViscousSolver::fused_pcg() const {
+  return prec_ != VecPrecond::NONE && prec_ != VecPrecond::BLOCK_JACOBI;
+}
+
+// As PoissonSolver::pcg_iterate, all components at once.
+PcgEnd VecViscousSolver::pcg_iterate(double tol, int limit) {
+  hipStream_t s = base_.stream_;
+  const int Np = base_.np();
+  const int64_t E = base_.mesh_.n_cells, stride = base_.stride_;
+  const int64_t cs = (int64_t)Np * stride, n = ncomp_ * cs;
+  double* const st = scal_.p + V_COUNT;
+  double* const part_pap = partial_.p;
+  double* const part_step = partial_.p + partial_.n / 2;
+  const double scale = prec_ == VecPrecond::FACTOR_INV_MASS ? base_.inv_mass_factor_ : 1.0;
+  const double* recp = prec_ == VecPrecond::RECP_FACTOR_DAT_INV_MASS ? base_.inv_mass_recp_.p : nullptr;
+  pcg_start(st, s);
+  auto step = [&](int k) {
+    const int rz = P_RZ0 + k % 2, rz_next = P_RZ0 + (k + 1) % 2;
+    Parts pap{part_pap, apply(p_.p, Ap_.p, part_pap)};
+    if (pap.n > kFoldParts) {
+      finalize(pap.n, 1, part_pap, st, P_SUM, s);
+      pap = Parts{st + P_SUM, 1};
+    }
+    const int nb = prec_ == VecPrecond::JACOBI
+                       ? pcg_update_jacobi(n, x_.p, r_.p, z_.p, p_.p, Ap_.p, inv_.p, pap, st, rz, part_step, s)
+                       : pcg_update_inv_mass(Np, ncomp_, E, stride, cs, x_.p, r_.p, z_.p, p_.p, Ap_.p, base_.J_.p,
+                                             minv_.p, scale, recp, pap, st, rz, part_step, s);
+    pcg_direction(n, p_.p, z_.p, nb, part_step, st, rz, rz_next, tol, s);
+  };
+  return pcg_drive(limit, n <= kAheadEntries, st, host_scal_ + V_COUNT, base_.ev_pcg_, s, step);
+}
+
 // ViscousSolver2D::solve (src/solvers/2d/slip_matrix/viscous_solver.cpp:59-75): boundary terms
 // into the rhs, then (preconditioned) CG over all components at once; inner products sum over
 // the components. As the scalar solve: flexible CG, true relative residual as the stopping test.
@@ -342,7 +392,6 @@ int VecViscousSolver::solve(const double* const rhs[], double* const ans[], Layo
   int status = 1, it = 0;
   double rr_true = 0;
   int64_t applies = 0;
-  const int nblk = ncomp_ * apply_blocks(E);
   if (!std::isfinite(bnorm)) {
     status = -3;
   } else {
@@ -357,11 +406,18 @@ int VecViscousSolver::solve(const double* const rhs[], double* const ans[], Layo
       if (std::sqrt(rr_true) <= tol) { status = 0; break; }
       if (it >= max_iter_ || restart > 50) { status = 1; break; }
       precondition(r_.p, z_.p);
-      dot<double>(n, r_.p, z_.p, nullptr, nullptr, 1, scal_.p, V_RZ, rs, s);
+      dot<double>(n, r_.p, z_.p, nullptr, nullptr, 1, scal_.p, fused_pcg() ? V_COUNT + P_RZ0 : V_RZ, rs, s);
       copy<double>(n, z_.p, p_.p, s);
+      if (fused_pcg()) {
+        const PcgEnd end = pcg_iterate(tol, max_iter_ - it);
+        it += end.iterations;
+        applies += end.iterations;
+        if (end.stop == PCG_BREAKDOWN) { status = -3; break; }
+        continue;
+      }
       bool breakdown = false;
       while (it < max_iter_) {
-        apply(p_.p, Ap_.p, partial_.p);  // p.Ap fused into the element passes
+        const int nblk = apply(p_.p, Ap_.p, partial_.p);  // p.Ap fused into the element passes
         ++applies;
         finalize(nblk, 1, partial_.p, scal_.p, V_PAP, s);
         cg_update_xr<double>(n, x_.p, r_.p, p_.p, Ap_.p, nullptr, nullptr, scal_.p, V_RZ, V_PAP, V_RR, rs, s);

@@ -55,7 +55,9 @@ class VecViscousSolver {
   int solve(const double* const rhs[], double* const ans[], Layout layout, SolveStats* stats);
 
  private:
-  void apply(const double* u, double* out, double* partial);
+  int apply(const double* u, double* out, double* partial);  // returns the partials of u.(A u) it leaves
+  bool fused_pcg() const;  // fused iterations (pcg_kernels.h)
+  PcgEnd pcg_iterate(double tol, int limit);
   void apply_one(int c, const double* u, double* out_c, double* partial);
   void precondition(const double* r, double* z);
   void build_block_jacobi();
