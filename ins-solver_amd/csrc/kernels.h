@@ -111,9 +111,10 @@ struct OiView {
   T* tU;
   T* tT;
 };
+// Returns the number of partials of u.(A u) it leaves (at most split_blocks(E), split_passes.h).
 template <typename T>
-void launch_apply_oi(const MeshView& m, const LevelView& l, const OiView<T>& o, const T* u, T* out,
-                     hipStream_t s, double* partial = nullptr);
+int launch_apply_oi(const MeshView& m, const LevelView& l, const OiView<T>& o, const T* u, T* out,
+                    hipStream_t s, double* partial = nullptr);
 void launch_diag_oi(const MeshView& m, const LevelView& l, const OiView<double>& o, double* diag,
                     hipStream_t s);
 // The kernels' compile-time rule sizes agree with the host's rule and tables.

@@ -194,6 +194,215 @@ k_apply_oi(int64_t E, int64_t stride, const T* __restrict__ u, const T* __restri
   }
 }
 
+// The same two passes with four waves to a cell (as sipg_split.h does for the nodal operator: 64 cells a
+// block, the waves' parts of A u meet in LDS): wave w takes face w, a share of the volume points that
+// balances the waves, and with them a quarter of the serial chain of an over-integrated cell (64 volume
+// and 24 face points at 3D order 2). The neighbour's point is fetched one point ahead. FP64 calls, one
+// thread per cell / four waves: 3D order 2, 29k cells 79.7 / 35.4 us, 1.05M 632 / 559; 3D order 3, 48k
+// 293 / 104, 664k 1410 / 1026; 3D order 4, 35k 724 / 360, 384k 2644 / 2103; 2D order 4, 20k 53.6 / 28.2,
+// 1.28M 584 / 589: the longer a cell's chain, the more even a full chip gains, so it is taken at every
+// size.
+template <int DIM, int N>
+struct OiShare {
+  int b[5];
+  constexpr OiShare() : b{} {
+    using L = OiL<DIM, N>;
+    const int col = 2 * DIM * L::Np, face = L::ns * L::Np * (DIM + 2);
+    int done = 0;
+    for (int w = 0; w < 4; ++w) {
+      b[w] = done;
+      const int faces_left = (L::Nf > w ? L::Nf - w : 0) * face;
+      int take = (((L::nv - done) * col + faces_left) / (4 - w) - (w < L::Nf ? face : 0) + col / 2) / col;
+      if (take < 0) take = 0;
+      if (w == 3 || done + take > L::nv) take = L::nv - done;
+      done += take;
+    }
+    b[4] = L::nv;
+  }
+};
+
+template <int DIM, int N, typename T>
+__global__ void __launch_bounds__(256)
+k_trace_oi_split(int64_t E, int64_t stride, const T* __restrict__ u, const double* __restrict__ Kt,
+                 const T* __restrict__ ks, const T* __restrict__ Cp, T* __restrict__ tU, T* __restrict__ tT) {
+  using L = OiL<DIM, N>;
+  constexpr int NK = DIM == 2 ? 3 : 6, NQ = L::Nf * L::ns;
+  const cptr<T> C = as_const(Cp);
+  const int64_t e = xcd_block() * 64 + (threadIdx.x & 63);
+  if (e >= E) return;
+  const int w = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  T uu[L::Np], K[NK];
+#pragma unroll
+  for (int m = 0; m < L::Np; ++m) uu[m] = u[m * stride + e];
+#pragma unroll
+  for (int k = 0; k < NK; ++k) K[k] = (T)Kt[k * stride + e];
+  // point g of the cell's Nf * ns, a quarter of them to a wave
+  for (int g = NQ * w / 4; g < NQ * (w + 1) / 4; ++g) {
+    const int f = g / L::ns, q = g - f * L::ns;
+    T beta[DIM];
+#pragma unroll
+    for (int s = 0; s < DIM; ++s) {
+      T b = 0;
+#pragma unroll
+      for (int r = 0; r < DIM; ++r) {
+        T al = 0;
+#pragma unroll
+        for (int k = 0; k < L::Nf; ++k) al = f == k ? (T)face_alpha(DIM, k, r) : al;
+        b = fma(al, K[kidx(DIM, r, s)], b);
+      }
+      beta[s] = b;
+    }
+    T U = 0, Tn = 0;
+#pragma unroll
+    for (int m = 0; m < L::Np; ++m) U = fma(C[L::off_IS + g * L::Np + m], uu[m], U);
+#pragma unroll
+    for (int s = 0; s < DIM; ++s) {
+      T d = 0;
+#pragma unroll
+      for (int m = 0; m < L::Np; ++m) d = fma(C[L::off_GS + ((f * DIM + s) * L::ns + q) * L::Np + m], uu[m], d);
+      Tn = fma(beta[s], d, Tn);
+    }
+    const int64_t idx = (int64_t)g * stride + e;
+    tU[idx] = U;
+    tT[idx] = ks[idx] * Tn;
+  }
+}
+
+template <int DIM, int N, typename T, int W>
+__device__ __forceinline__ void
+oi_quarter(int64_t e, int64_t stride, const T* __restrict__ u, const T* __restrict__ tU,
+           const T* __restrict__ tT, const double* __restrict__ Kt, const double* __restrict__ tauS,
+           const int* __restrict__ nbr, const int* __restrict__ bctype, const T* __restrict__ kv,
+           const T* __restrict__ ks, cptr<T> C, cptr<int> qmap, T (&acc)[OiL<DIM, N>::Np]) {
+  using L = OiL<DIM, N>;
+  constexpr int NK = DIM == 2 ? 3 : 6;
+  constexpr OiShare<DIM, N> share;
+  constexpr bool has_face = W < L::Nf;
+  constexpr int F0 = has_face ? W : 0;
+  int nb = 0;
+  T ts = 0;
+  if constexpr (has_face) {
+    nb = nbr[F0 * stride + e];
+    ts = (T)tauS[F0 * stride + e];
+  }
+  T uu[L::Np], K[NK];
+#pragma unroll
+  for (int m = 0; m < L::Np; ++m) {
+    uu[m] = u[m * stride + e];
+    acc[m] = 0;
+  }
+#pragma unroll
+  for (int k = 0; k < NK; ++k) K[k] = (T)Kt[k * stride + e];
+  int mode = 2;  // 0 interior, 1 Dirichlet, 2 no terms
+  int64_t own = 0, nbase = 0;
+  cptr<int> map = qmap;
+  if constexpr (has_face) {
+    mode = nb >= 0 ? 0 : (bctype[-nb - 1] == 0 ? 1 : 2);
+    const int c = nb & 31, fn = nb >= 0 ? c / L::nperm : F0, p = nb >= 0 ? c - fn * L::nperm : 0;
+    own = (int64_t)F0 * L::ns * stride + e;
+    nbase = (int64_t)fn * L::ns * stride + (nb >= 0 ? (int64_t)(nb >> 5) : e);
+    map = qmap + p * L::ns;
+  }
+  // values of the first face point, in flight during the volume term
+  T Um = 0, Tm = 0, Up = 0, Tp = 0, kq = 0;
+  auto fetch = [&](int q) {
+    const int64_t n = nbase + (int64_t)map[q] * stride, o = own + (int64_t)q * stride;
+    Um = tU[o];
+    Tm = tT[o];
+    kq = ks[o];
+    Up = tU[n];
+    Tp = tT[n];
+  };
+  if constexpr (has_face) fetch(0);
+  T kn = share.b[W] < share.b[W + 1] ? kv[(int64_t)share.b[W] * stride + e] : (T)0;
+#pragma unroll 1
+  for (int q = share.b[W]; q < share.b[W + 1]; ++q) {
+    const T wk = C[L::off_wv + q] * kn;
+    kn = kv[(int64_t)(q + 1 < share.b[W + 1] ? q + 1 : q) * stride + e];
+    T g[DIM];
+#pragma unroll
+    for (int s = 0; s < DIM; ++s) {
+      T a = 0;
+#pragma unroll
+      for (int m = 0; m < L::Np; ++m) a = fma(C[L::off_GV + (s * L::nv + q) * L::Np + m], uu[m], a);
+      g[s] = a;
+    }
+#pragma unroll
+    for (int r = 0; r < DIM; ++r) {
+      T h = 0;
+#pragma unroll
+      for (int s = 0; s < DIM; ++s) h = fma(K[kidx(DIM, r, s)], g[s], h);
+      h *= wk;
+#pragma unroll
+      for (int i = 0; i < L::Np; ++i) acc[i] = fma(C[L::off_GV + (r * L::nv + q) * L::Np + i], h, acc[i]);
+    }
+  }
+  if constexpr (has_face) {
+    if (mode == 2) return;
+    T beta[DIM];
+    face_beta<DIM>(K, F0, beta);
+#pragma unroll 1
+    for (int q = 0; q < L::ns; ++q) {
+      const T um = Um, tm = Tm, k = kq;
+      const T up = mode == 0 ? Up : -um, tp = mode == 0 ? Tp : -tm;
+      fetch(q + 1 < L::ns ? q + 1 : q);
+      const T wq = C[L::off_ws + q];
+      const T jump = um - up;
+      const T F = wq * (T)0.5 * (ts * jump - (tm - tp));
+      const T sig = wq * (T)-0.5 * k * jump;
+      T bs[DIM];
+#pragma unroll
+      for (int s = 0; s < DIM; ++s) bs[s] = beta[s] * sig;
+#pragma unroll
+      for (int i = 0; i < L::Np; ++i) {
+        T a = fma(C[L::off_IS + (F0 * L::ns + q) * L::Np + i], F, acc[i]);
+#pragma unroll
+        for (int s = 0; s < DIM; ++s) a = fma(C[L::off_GS + ((F0 * DIM + s) * L::ns + q) * L::Np + i], bs[s], a);
+        acc[i] = a;
+      }
+    }
+  }
+}
+
+template <int DIM, int N, typename T>
+__global__ void __launch_bounds__(256)
+k_apply_oi_split(int64_t E, int64_t stride, const T* __restrict__ u, const T* __restrict__ tU,
+                 const T* __restrict__ tT, const double* __restrict__ Kt, const double* __restrict__ tauS,
+                 const int* __restrict__ nbr, const int* __restrict__ bctype, const T* __restrict__ kv,
+                 const T* __restrict__ ks, const T* __restrict__ Cp, const int* __restrict__ qmapp,
+                 T* __restrict__ out, double* __restrict__ partial) {
+  using L = OiL<DIM, N>;
+  __shared__ T part[4][L::Np][64];
+  const cptr<T> C = as_const(Cp);
+  const cptr<int> qmap = as_const(qmapp);
+  const int w = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int64_t e = xcd_block() * 64 + lane;
+  if (e < E) {
+    T acc[L::Np];
+    switch (w) {
+      case 0: oi_quarter<DIM, N, T, 0>(e, stride, u, tU, tT, Kt, tauS, nbr, bctype, kv, ks, C, qmap, acc); break;
+      case 1: oi_quarter<DIM, N, T, 1>(e, stride, u, tU, tT, Kt, tauS, nbr, bctype, kv, ks, C, qmap, acc); break;
+      case 2: oi_quarter<DIM, N, T, 2>(e, stride, u, tU, tT, Kt, tauS, nbr, bctype, kv, ks, C, qmap, acc); break;
+      default: oi_quarter<DIM, N, T, 3>(e, stride, u, tU, tT, Kt, tauS, nbr, bctype, kv, ks, C, qmap, acc); break;
+    }
+#pragma unroll
+    for (int i = 0; i < L::Np; ++i) part[w][i][lane] = acc[i];
+  }
+  __syncthreads();
+  double dotv = 0.0;
+  if (e < E) {
+    for (int i = w; i < L::Np; i += 4) {
+      const T a = (part[0][i][lane] + part[1][i][lane]) + (part[2][i][lane] + part[3][i][lane]);
+      out[i * stride + e] = a;
+      dotv += (double)u[i * stride + e] * (double)a;
+    }
+  }
+  if (partial) {
+    const double t = block_sum1<256>(dotv);
+    if (threadIdx.x == 0) partial[blockIdx.x] = t;
+  }
+}
+
 // Exact diagonal of the over-integrated operator.
 template <int DIM, int N>
 __global__ void __launch_bounds__(256)
@@ -273,9 +482,23 @@ bool oi_shape_matches(int dim, int N, int nv, int ns, int table_size) {
 }
 
 template <typename T>
-void launch_apply_oi(const MeshView& m, const LevelView& l, const OiView<T>& o, const T* u, T* out,
-                     hipStream_t s, double* partial) {
-  if (m.E == 0) return;
+int launch_apply_oi(const MeshView& m, const LevelView& l, const OiView<T>& o, const T* u, T* out,
+                    hipStream_t s, double* partial) {
+  if (m.E == 0) return 0;
+  // four waves to a cell wherever the neighbour words are packed (meshes below 2^26 cells)
+  if (m.nbc) {
+    const dim3 grid((unsigned)((m.E + 63) / 64));
+    INSP_OI_DISPATCH(m.dim, l.N,
+                     hipLaunchKernelGGL((k_trace_oi_split<D_, N_, T>), grid, dim3(256), 0, s, m.E, m.stride, u,
+                                        m.Kt, o.ks, o.C, o.tU, o.tT));
+    check("k_trace_oi_split");
+    INSP_OI_DISPATCH(m.dim, l.N,
+                     hipLaunchKernelGGL((k_apply_oi_split<D_, N_, T>), grid, dim3(256), 0, s, m.E, m.stride, u,
+                                        o.tU, o.tT, m.Kt, l.tauS, m.nbc, m.bctype, o.kv, o.ks, o.C, o.qmap, out,
+                                        partial));
+    check("k_apply_oi_split");
+    return (int)grid.x;
+  }
   INSP_OI_DISPATCH(m.dim, l.N,
                    hipLaunchKernelGGL((k_trace_oi<D_, N_, T>), grid_oi(m.E), dim3(256), 0, s, m.E, m.stride, u,
                                       m.Kt, o.ks, o.C, o.tU, o.tT));
@@ -285,6 +508,7 @@ void launch_apply_oi(const MeshView& m, const LevelView& l, const OiView<T>& o, 
                                       o.tU, o.tT, m.Kt, l.tauS, m.nbr, m.code, m.bctype, o.kv, o.ks, o.C,
                                       o.qmap, out, partial));
   check("k_apply_oi");
+  return apply_blocks(m.E);
 }
 
 void launch_diag_oi(const MeshView& m, const LevelView& l, const OiView<double>& o, double* diag,
@@ -296,9 +520,9 @@ void launch_diag_oi(const MeshView& m, const LevelView& l, const OiView<double>&
   check("k_diag_oi");
 }
 
-template void launch_apply_oi<double>(const MeshView&, const LevelView&, const OiView<double>&, const double*,
-                                      double*, hipStream_t, double*);
-template void launch_apply_oi<float>(const MeshView&, const LevelView&, const OiView<float>&, const float*,
-                                     float*, hipStream_t, double*);
+template int launch_apply_oi<double>(const MeshView&, const LevelView&, const OiView<double>&, const double*,
+                                     double*, hipStream_t, double*);
+template int launch_apply_oi<float>(const MeshView&, const LevelView&, const OiView<float>&, const float*,
+                                    float*, hipStream_t, double*);
 
 }  // namespace insp

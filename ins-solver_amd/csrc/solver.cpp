@@ -752,7 +752,7 @@ int PoissonSolver::apply_level(int l, const T* u, T* out, double* partial, T* tr
     launch_apply_p1_cells<T>(mv, v, u, k, out, stream_, partial);
   } else if (oi_ && l == 0) {
     if (prof) INSP_HIP(hipEventRecord(e1, stream_));
-    launch_apply_oi<T>(mv, v, oi_view<T>(), u, out, stream_, partial);
+    npart = launch_apply_oi<T>(mv, v, oi_view<T>(), u, out, stream_, partial);
   } else if (!v.frag && split_apply(mv, v, std::is_same<T, float>::value)) {
     trace_pass<T>(mv, v, u, k, tr, stream_);
     if (prof) INSP_HIP(hipEventRecord(e1, stream_));

@@ -95,3 +95,31 @@ def test_coarse_cg_forms(ip, oracle, dim, n, iters, mixed, factor):
     assert np.linalg.norm(b - o.mult(x)) <= 2e-9 * np.linalg.norm(b)
     assert s.solve(b, y) and s.last_stats["iterations"] == its
     assert np.array_equal(x, y)
+
+
+@pytest.mark.parametrize("dim,N,n", [(2, 1, 1), (2, 2, 6), (2, 3, 7), (2, 4, 9), (3, 1, 3), (3, 2, 1), (3, 3, 3),
+                                     (3, 4, 2)])
+def test_over_integrated_apply(ip, oracle, dim, N, n):
+    """Remainders of the 64-cell blocks, mixed boundary types, both precisions (tolerances as above; the
+    face and volume sums have at most 216 + 64 terms)."""
+    mesh = ip.Mesh.square(n, jitter=0.1, seed=6) if dim == 2 else ip.Mesh.cube(n, 0.1, 6)
+    s = ip.PoissonSolver(mesh, N)
+    o = oracle.Oracle(*mesh.arrays(), N, faces=mesh.faces())
+    bt = np.zeros(s.n_bfaces, dtype=np.int32)
+    bt[1::3] = 1
+    s.set_bc_types(bt)
+    o.set_bc_types(bt)
+    rule = ip.oi_rule(dim, N)
+    rng = np.random.default_rng(n)
+    kv = 1.0 + rng.random((s.n_cells, rule[0].shape[0]))
+    ks = 1.0 + rng.random((s.n_cells, (dim + 1) * rule[2].shape[0]))
+    kn = 1.0 + rng.random((s.n_cells, s.Np))
+    s.set_factor(kn)
+    o.set_factor(kn)
+    s.set_factor_oi(kv)
+    s.set_factor_surf_oi(ks)
+    s.set_solver(ip.SOLVER_JACOBI)
+    x = rng.standard_normal((s.n_cells, s.Np))
+    y = o.mult_oi(rule, kv, ks, x)
+    assert rel(s.mult(x), y) < (1e-12 if N < 4 else 1e-11)
+    assert rel(s.mult_fp32(x), y) < 2e-5
