@@ -155,15 +155,14 @@ struct ChebOut {
   }
 };
 
-// Face nodes per load round of the element pass (a divisor of Nfp): whole faces where the
-// registers allow it (2D, and 3D up to order 3 in FP32 and order 2 in FP64). 3D faces of order 4,
-// and of order 3 in FP64, go one node at a time: larger rounds cost a wave per SIMD and measured
-// slower (64^3x6 tets, FP64 order 3: 731 us per element pass one node at a time, 774 us two at a
-// time, 1021 us whole faces; 48^3x6, FP64 order 4: 1116 us one at a time, 1322 us five).
-constexpr int face_chunk(int dim, int N, int bytes) {
-  const int nfp = dim == 2 ? N + 1 : (N + 1) * (N + 2) / 2;
-  if (dim == 3 && (N == 4 || (N == 3 && bytes == 8))) return 1;
-  return nfp;
+// Whether the element pass loads a whole face at a time: 2D, and 3D up to order 3 in FP32 and order 2 in
+// FP64. 3D faces of order 4, and of order 3 in FP64, go one node at a time: larger rounds cost a wave
+// per SIMD and measured slower (64^3x6 tets, FP64 order 3: 731 us per element pass one node at a
+// time, 774 us two at a time, 1021 us whole faces; 48^3x6, FP64 order 4: 1116 us one at a time, 1322
+// us five). With the loads of a node issued a node ahead: FP64 order 3, 384,000 cells 184 -> 161 us,
+// 64^3x6 745 -> 666 us; order 4, 384,000 cells 584 -> 534 us.
+constexpr bool whole_faces(int dim, int N, int bytes) {
+  return !(dim == 3 && (N == 4 || (N == 3 && bytes == 8)));
 }
 
 // One cell of the element pass; returns u.(A u) over the cell. PACK: nbr holds the packed
@@ -229,14 +228,12 @@ apply_cell(int64_t e, int64_t stride, const T* __restrict__ u, const T* __restri
     if constexpr (MASS) mc.add(j, Np, C + L.off_M + j * Np, acc);
   }
 
-  // Face terms. The face nodes are taken in chunks of CH; the loads of a chunk are issued in
-  // two rounds before its arithmetic: the cell's own traces with the node map of the shared
-  // face, then the neighbour's values and traces at the mapped nodes. A boundary face reads
-  // the cell's own entries in the second round and does not use them. With one chunk per face
-  // the loops unroll completely and the cell's own face-node values come from registers.
-  constexpr int CH = face_chunk(DIM, N, (int)sizeof(T));
-  static_assert(Nfp % CH == 0, "face chunks");
-  constexpr bool whole = CH == Nfp;
+  // Face terms. Where the registers allow it a face's loads are issued in two rounds before its
+  // arithmetic: the cell's own traces with the node map of the shared face, then the neighbour's
+  // values and traces at the mapped nodes; the loops unroll completely and the cell's own face-node
+  // values come from registers. Otherwise the nodes go one at a time. A boundary face reads the
+  // cell's own entries in the second round and does not use them.
+  constexpr bool whole = whole_faces(DIM, N, (int)sizeof(T));
 #pragma unroll
   for (int f = 0; f < Nf; ++f) {
     T beta[DIM];
@@ -265,69 +262,86 @@ apply_cell(int64_t e, int64_t stride, const T* __restrict__ u, const T* __restri
     T sv[Nfp];
 #pragma unroll
     for (int i = 0; i < Nfp; ++i) sv[i] = 0;
-    auto chunk = [&](int j0) {
-      T Tm[CH], up[CH], Tp[CH], um[CH];
-      int pk[CH];
+    // the terms of face node j (volume node p): own and neighbour's value and trace, own coefficient
+    auto node = [&](int j, int p, T umj, T tm, T up, T Tp, T kp) {
+      if constexpr (Slip::enabled) {
+        if (mode == 3) {
+          const double* n = slip.bn + (int64_t)(-nb - 1) * DIM;
+          T su = 0, st = 0;
 #pragma unroll
-      for (int jj = 0; jj < CH; ++jj) {
-        const int j = j0 + jj;
-        Tm[jj] = tr[(int64_t)(f * Nfp + j) * stride + e];
-        pk[jj] = tab[tbase + j];
-        if constexpr (whole) um[jj] = uu[FM.v[f * Nfp + j]];
-        else um[jj] = u[tab[L.tab_fmask + f * Nfp + j] * stride + e];
-      }
-#pragma unroll
-      for (int jj = 0; jj < CH; ++jj) {
-        up[jj] = u[(int64_t)(pk[jj] >> 6) * stride + q];
-        Tp[jj] = tr[(int64_t)(pk[jj] & 63) * stride + q];
-      }
-#pragma unroll
-      for (int jj = 0; jj < CH; ++jj) {
-        const int j = j0 + jj;
-        const int p = whole ? FM.v[f * Nfp + j] : tab[L.tab_fmask + f * Nfp + j];
-        T umj = um[jj];
-        T tm = Tm[jj];
-        if constexpr (Slip::enabled) {
-          if (mode == 3) {
-            const double* n = slip.bn + (int64_t)(-nb - 1) * DIM;
-            T su = 0, st = 0;
-#pragma unroll
-            for (int d = 0; d < DIM; ++d) {
-              su = fma((T)n[d], slip.u0[d * slip.cstride + p * stride + e], su);
-              st = fma((T)n[d], slip.tr0[d * slip.tstride + (int64_t)(f * Nfp + j) * stride + e], st);
-            }
-            umj = (T)n[slip.comp] * su;
-            tm = (T)n[slip.comp] * st;
+          for (int d = 0; d < DIM; ++d) {
+            su = fma((T)n[d], slip.u0[d * slip.cstride + p * stride + e], su);
+            st = fma((T)n[d], slip.tr0[d * slip.tstride + (int64_t)(f * Nfp + j) * stride + e], st);
           }
+          umj = (T)n[slip.comp] * su;
+          tm = (T)n[slip.comp] * st;
         }
-        const T upj = mode == 0 ? up[jj] : -umj;
-        const T tpj = mode == 0 ? Tp[jj] : -tm;
-        const T jump = umj - upj;
-        const T F = (T)0.5 * (ts * jump - (tm - tpj));
-        T sig = (T)-0.5 * jump;
-        sig *= kval<VAR>(kfac, p * stride + e);
+      }
+      const T upj = mode == 0 ? up : -umj;
+      const T tpj = mode == 0 ? Tp : -tm;
+      const T jump = umj - upj;
+      const T F = (T)0.5 * (ts * jump - (tm - tpj));
+      T sig = (T)-0.5 * jump;
+      sig *= kp;
 #pragma unroll
-        for (int i = 0; i < Nfp; ++i) {
-          const T mf = C[L.off_MfT + (f * Nfp + j) * Nfp + i];
-          acc[FM.v[f * Nfp + i]] = fma(mf, F, acc[FM.v[f * Nfp + i]]);
-          if constexpr (fold) sv[i] = fma(mf, sig, sv[i]);
-        }
-        if constexpr (!fold) {
+      for (int i = 0; i < Nfp; ++i) {
+        const T mf = C[L.off_MfT + (f * Nfp + j) * Nfp + i];
+        acc[FM.v[f * Nfp + i]] = fma(mf, F, acc[FM.v[f * Nfp + i]]);
+        if constexpr (fold) sv[i] = fma(mf, sig, sv[i]);
+      }
+      if constexpr (!fold) {
 #pragma unroll
-          for (int r = 0; r < DIM; ++r) {
-            const T bs = beta[r] * sig;
+        for (int r = 0; r < DIM; ++r) {
+          const T bs = beta[r] * sig;
 #pragma unroll
-            for (int i = 0; i < Np; ++i)
-              acc[i] = fma(C[L.off_Wt + ((f * DIM + r) * Nfp + j) * Np + i], bs, acc[i]);
-          }
+          for (int i = 0; i < Np; ++i)
+            acc[i] = fma(C[L.off_Wt + ((f * DIM + r) * Nfp + j) * Np + i], bs, acc[i]);
         }
       }
     };
     if constexpr (whole) {
-      chunk(0);
+      T Tm[Nfp], up[Nfp], Tp[Nfp];
+      int pk[Nfp];
+#pragma unroll
+      for (int j = 0; j < Nfp; ++j) {
+        Tm[j] = tr[(int64_t)(f * Nfp + j) * stride + e];
+        pk[j] = tab[tbase + j];
+      }
+#pragma unroll
+      for (int j = 0; j < Nfp; ++j) {
+        up[j] = u[(int64_t)(pk[j] >> 6) * stride + q];
+        Tp[j] = tr[(int64_t)(pk[j] & 63) * stride + q];
+      }
+#pragma unroll
+      for (int j = 0; j < Nfp; ++j)
+        node(j, FM.v[f * Nfp + j], uu[FM.v[f * Nfp + j]], Tm[j], up[j], Tp[j],
+             kval<VAR>(kfac, FM.v[f * Nfp + j] * stride + e));
     } else {
+      // one node at a time, its loads issued during the node before and the node map's entry during the
+      // one before that
+      struct Node {
+        int p;
+        T um, Tm, up, Tp, k;
+      };
+      auto load = [&](int j, int pk) {
+        Node x;
+        x.p = tab[L.tab_fmask + f * Nfp + j];
+        x.um = u[x.p * stride + e];
+        x.Tm = tr[(int64_t)(f * Nfp + j) * stride + e];
+        x.k = kval<VAR>(kfac, x.p * stride + e);
+        x.up = u[(int64_t)(pk >> 6) * stride + q];
+        x.Tp = tr[(int64_t)(pk & 63) * stride + q];
+        return x;
+      };
+      Node cur = load(0, tab[tbase]);
+      int pk = tab[tbase + 1];
 #pragma unroll 1
-      for (int j0 = 0; j0 < Nfp; j0 += CH) chunk(j0);
+      for (int j = 0; j < Nfp; ++j) {
+        const Node nxt = load(j + 1 < Nfp ? j + 1 : j, pk);
+        pk = tab[tbase + (j + 2 < Nfp ? j + 2 : Nfp - 1)];
+        node(j, cur.p, cur.um, cur.Tm, cur.up, cur.Tp, cur.k);
+        cur = nxt;
+      }
     }
     // symmetry term sum_r beta_r D_r^T (EMAT_f sig): the face mass first, then the rows
     // of D_r at the face nodes
