@@ -111,6 +111,7 @@ k_apply_mfma(int64_t E, int64_t stride, const float* __restrict__ u, const float
   const T* f1 = fr;
   const T* f2 = fr + S::F1 * 64;
   const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int waves = blockDim.x >> 6;
   const int g = lane >> 4, c = lane & 15;
   const uint32_t st = (uint32_t)stride;
 
@@ -123,8 +124,8 @@ k_apply_mfma(int64_t E, int64_t stride, const float* __restrict__ u, const float
   const int nbx = nb_all / nx + (x < nb_all % nx ? 1 : 0);
   const int64_t t_end = ntiles * (x + 1) / nx;
 #pragma unroll 1
-  for (int64_t tile = ntiles * x / nx + (int64_t)(b / nx) * S::WAVES + w; tile < t_end;
-       tile += (int64_t)nbx * S::WAVES) {
+  for (int64_t tile = ntiles * x / nx + (int64_t)(b / nx) * waves + w; tile < t_end;
+       tile += (int64_t)nbx * waves) {
     const int64_t e = tile * 16 + c;
     const bool live = e < E;
     const uint32_t ec = (uint32_t)e;
@@ -284,10 +285,22 @@ void launch_order(const MeshView& m, const LevelView& l, const float* u, const f
   // 32-bit element offsets: the largest array indexed is the trace, Nf*Nfp rows
   if ((int64_t)SH::Nf * SH::Nfp * m.stride * (int64_t)sizeof(double) >= (int64_t(1) << 32))
     throw std::runtime_error("matrix-core element pass: mesh too large for 32-bit offsets");
-  const int64_t groups = (((m.E + 15) / 16) + SH::WAVES - 1) / SH::WAVES;
+  const int64_t tiles = (m.E + 15) / 16;
+  const int64_t groups = (tiles + SH::WAVES - 1) / SH::WAVES;
   const int res = resident_blocks((const void*)k_apply_mfma<N, VAR>, SH::WAVES * 64, N, VAR ? 1 : 0);
-  const dim3 grid((unsigned)std::min<int64_t>(groups, res));
-  hipLaunchKernelGGL((k_apply_mfma<N, VAR>), grid, dim3(SH::WAVES * 64), 0, s, m.E, m.stride, u, tr,
+  int64_t blocks = std::min<int64_t>(groups, res);
+  int waves = SH::WAVES;
+  if (N == 4 && groups <= res && res % 8 == 0) {
+    // One tile per wave and CUs to spare: as many waves per block (one block fits a CU) as give every
+    // CU its share of an XCD's tiles, four at least to load the fragments. us per pass with 16 waves
+    // / this: 6,000 cells 31.2 / 19.4, 48,000 48.6 / 31.8, 63,888 45.9 / 36.9 (with a coefficient).
+    const int64_t per_xcd = (tiles + 7) / 8;
+    const int64_t bx = std::min<int64_t>(res / 8, (per_xcd + 3) / 4);
+    waves = (int)std::max<int64_t>(4, (per_xcd + bx - 1) / bx);
+    blocks = 8 * bx;
+  }
+  const dim3 grid((unsigned)blocks);
+  hipLaunchKernelGGL((k_apply_mfma<N, VAR>), grid, dim3(waves * 64), 0, s, m.E, m.stride, u, tr,
                      m.Kt, l.tauS, m.nbr, m.code, m.bctype, kfac,
                      static_cast<const float*>(l.frag), l.tab, out);
 }
