@@ -256,17 +256,29 @@ k_p1_direction(int64_t E, int64_t stride, const T* __restrict__ z, const T* __re
   put_partial(dotv, partial);
 }
 
-// Pairs per thread of the streams: one while that leaves few enough partials to fold, else two.
-int per_thread(int64_t n2) { return n2 <= (int64_t)kBlock * kFoldParts ? 1 : 2; }
+// Pairs per thread of the streams: one, two or four while that leaves about a thousand blocks, whose
+// partials (and their reading of others') are cheap; longer vectors stream at two per thread and leave
+// the partials to a kernel in between. us per coarse iteration, 3D order 1: 547k cells with two per
+// thread and finalize 57.3, four and folded 54.5; 1.57M cells 157.4, eight and folded 161.1.
+int per_thread(int64_t n2) {
+  if (n2 <= (int64_t)kBlock * 1024) return 1;
+  if (n2 <= (int64_t)kBlock * 2 * 1024 || n2 > (int64_t)kBlock * 4 * 1536) return 2;
+  return 4;
+}
 int blocks(int64_t n2, int per) { return (int)((n2 + (int64_t)kBlock * per - 1) / ((int64_t)kBlock * per)); }
 
 }  // namespace
 
 #define INSP_PER(n2, CALL)                       \
   do {                                           \
-    if (per_thread(n2) == 1) { constexpr int P_ = 1; CALL; } \
-    else { constexpr int P_ = 2; CALL; }         \
+    switch (per_thread(n2)) {                    \
+      case 1: { constexpr int P_ = 1; CALL; } break; \
+      case 2: { constexpr int P_ = 2; CALL; } break; \
+      default: { constexpr int P_ = 4; CALL; }   \
+    }                                            \
   } while (0)
+
+int cg_stream_blocks(int64_t n) { return blocks(n / 2, per_thread(n / 2)); }
 
 template <typename T>
 int cg_init(int64_t n, const T* b, const T* inv, T* x, T* z, T* p, double* partial, hipStream_t s) {

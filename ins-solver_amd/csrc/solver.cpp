@@ -922,8 +922,9 @@ void PoissonSolver::coarse_cg(int l) {
   // are too many for that, as one value added up by a kernel in between.
   double* const part_pap = partial_.p;
   double* const part_rz = partial_.p + partial_.n / 2;
+  const int consumer = cg_stream_blocks(n);
   auto folded = [&](int np, double* part, int slot) {
-    if (np <= kFoldParts) return Parts{part, np};
+    if (fold_pays(np, consumer)) return Parts{part, np};
     finalize(np, 1, part, scal_.p, slot, stream_);
     return Parts{scal_.p + slot, 1};
   };
