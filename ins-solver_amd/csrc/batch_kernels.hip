@@ -100,12 +100,9 @@ __device__ __forceinline__ Cell locate_order(const BatchView& b) {
   return c;
 }
 
-// Face traces of order-NN problems (order 1 needs none).
-template <int TB, int DIM, typename T, int NN>
-__global__ void __launch_bounds__(TB) kb_trace(BatchView b, BatchTables tb, int in, int tr) {
-  const Cell c = locate_order<TB, NN>(b);
-  if (!c.live) return;  // uniform per block
-  const BatchProb& P = b.P[c.slot];
+// Face traces of one cell of an order-NN problem (order 1 needs none).
+template <int DIM, typename T, int NN>
+__device__ __forceinline__ void trace_tile(const BatchTables& tb, const Cell& c, const BatchProb& P, int in, int tr) {
   const int prec = std::is_same<T, float>::value;
   const int64_t S = uni(P.S);
   const T* u = uni((const T*)P.v[in]);
@@ -117,38 +114,86 @@ __global__ void __launch_bounds__(TB) kb_trace(BatchView b, BatchTables tb, int 
   trace_cell<DIM, NN, T, 2>(c.e, S, u, Kt, k, as_const(C), trp);
 }
 
+// Operator on one cell of an order-NN problem, on its own order or (LEVEL1) on order 1.
+template <int DIM, typename T, int NN, bool LEVEL1>
+__device__ __forceinline__ double apply_tile(const BatchTables& tb, const Cell& c, const BatchProb& P, int in, int tr,
+                                             int out) {
+  const int prec = std::is_same<T, float>::value;
+  const int64_t S = uni(P.S);
+  const T* u = uni((const T*)P.v[in]);
+  T* o = uni((T*)P.v[out]);
+  const double* tau = uni(LEVEL1 ? P.tauC : P.tauF);
+  const T* k = uni((const T*)(LEVEL1 ? P.kC[prec] : P.kF[prec]));
+  const T* C = uni(ctab<T>(tb, NN));
+  const int* tab = uni(tb.tab[NN]);
+  const double* Kt = uni(P.Kt);
+  const int* nbr = uni(P.nbr);
+  const int* code = uni(P.code);
+  const int* bct = uni(P.bctype);
+  if (!c.valid) return 0.0;
+  if constexpr (NN == 1) {
+    return apply_p1_cell<DIM, T, 2>(c.e, S, u, Kt, tau, nbr, code, bct, k, as_const(C), as_const(tab), o);
+  } else {
+    const T* trp = uni((const T*)P.v[tr]);
+    return apply_cell<DIM, NN, T, 2>(c.e, S, u, trp, Kt, tau, nbr, code, bct, k, as_const(C), as_const(tab), o);
+  }
+}
+
+// Order-NN problems, one order per kernel so each is compiled lean.
+template <int TB, int DIM, typename T, int NN>
+__global__ void __launch_bounds__(TB) kb_trace(BatchView b, BatchTables tb, int in, int tr) {
+  const Cell c = locate_order<TB, NN>(b);
+  if (!c.live) return;  // uniform per block
+  trace_tile<DIM, T, NN>(tb, c, b.P[c.slot], in, tr);
+}
+
 // Operator of order-NN problems on their own order (level 0); with LEVEL1 the order-1
-// operator of every problem (all tiles), one order per kernel so each is compiled lean.
+// operator of every problem (all tiles), again one order per kernel.
 template <int TB, int DIM, typename T, int NN, bool LEVEL1>
 __global__ void __launch_bounds__(TB)
 kb_apply(BatchView b, BatchTables tb, int in, int tr, int out, int dot) {
   const Cell c = LEVEL1 ? locate<TB>(b) : locate_order<TB, NN>(b);
   double dv[1] = {0.0};
-  if (c.live) {  // uniform per block: the problem's data in scalar registers
+  if (c.live)  // uniform per block: the problem's data in scalar registers
+    dv[0] = apply_tile<DIM, T, NN, LEVEL1>(tb, c, b.P[c.slot], in, tr, out);
+  if (dot) put_partials<TB, 1>(b, c, dv);
+}
+
+// Every order in one launch, for batches of few tiles. Such a batch does not fill the chip, and
+// the one-order launches run one after the other, each as long as one tile's own chain of loads
+// and products whatever its number of tiles; here they run side by side and the launch lasts as
+// long as its highest order. It holds that order's registers for every tile, so a batch that
+// fills the chip keeps the launches by order (launch_all_orders).
+constexpr int kAllTile = 64;
+
+template <int DIM, typename T>
+__global__ void __launch_bounds__(kAllTile) kb_trace_all(BatchView b, BatchTables tb, int in, int tr) {
+  const Cell c = locate<kAllTile>(b);
+  if (!c.live) return;  // uniform per block
+  const BatchProb& P = b.P[c.slot];
+  switch (uni(P.N)) {
+    case 2: trace_tile<DIM, T, 2>(tb, c, P, in, tr); break;
+    case 3: trace_tile<DIM, T, 3>(tb, c, P, in, tr); break;
+    case 4: trace_tile<DIM, T, 4>(tb, c, P, in, tr); break;
+    default: break;
+  }
+}
+
+template <int DIM, typename T>
+__global__ void __launch_bounds__(kAllTile)
+kb_apply_all(BatchView b, BatchTables tb, int in, int tr, int out, int dot) {
+  const Cell c = locate<kAllTile>(b);
+  double dv[1] = {0.0};
+  if (c.live) {
     const BatchProb& P = b.P[c.slot];
-    const int prec = std::is_same<T, float>::value;
-    const int64_t S = uni(P.S);
-    const T* u = uni((const T*)P.v[in]);
-    T* o = uni((T*)P.v[out]);
-    const double* tau = uni(LEVEL1 ? P.tauC : P.tauF);
-    const T* k = uni((const T*)(LEVEL1 ? P.kC[prec] : P.kF[prec]));
-    const T* C = uni(ctab<T>(tb, NN));
-    const int* tab = uni(tb.tab[NN]);
-    const double* Kt = uni(P.Kt);
-    const int* nbr = uni(P.nbr);
-    const int* code = uni(P.code);
-    const int* bct = uni(P.bctype);
-    if (c.valid) {
-      if constexpr (NN == 1) {
-        dv[0] = apply_p1_cell<DIM, T, 2>(c.e, S, u, Kt, tau, nbr, code, bct, k, as_const(C), as_const(tab), o);
-      } else {
-        const T* trp = uni((const T*)P.v[tr]);
-        dv[0] = apply_cell<DIM, NN, T, 2>(c.e, S, u, trp, Kt, tau, nbr, code, bct, k, as_const(C), as_const(tab),
-                                          o);
-      }
+    switch (uni(P.N)) {
+      case 1: dv[0] = apply_tile<DIM, T, 1, false>(tb, c, P, in, tr, out); break;
+      case 2: dv[0] = apply_tile<DIM, T, 2, false>(tb, c, P, in, tr, out); break;
+      case 3: dv[0] = apply_tile<DIM, T, 3, false>(tb, c, P, in, tr, out); break;
+      default: dv[0] = apply_tile<DIM, T, 4, false>(tb, c, P, in, tr, out); break;
     }
   }
-  if (dot) put_partials<TB, 1>(b, c, dv);
+  if (dot) put_partials<kAllTile, 1>(b, c, dv);
 }
 
 __global__ void __launch_bounds__(kB) kb_finalize(BatchView b, int nvals, int slot0) {
@@ -684,8 +729,24 @@ dim3 tiles_grid(const BatchView& b) { return dim3((unsigned)b.tile_cap); }
     else { constexpr int D_ = 3; CALL; }    \
   } while (0)
 
+// All orders in one launch (kb_trace_all, kb_apply_all) while the grid is at most this many 64-cell
+// tiles; the line lies where the chip is filled by one wave per tile holding the highest order's
+// registers. Measured per lockstep iteration, problems of orders 2-4, launches by order -> one
+// launch: 2D mixed precision, 253 tiles 577 -> 413 us, 1518 900 -> 670, 3037 (a grid of 4096)
+// 1100 -> 935; 2D FP64, 3037 tiles 1280 -> 1094. 3D mixed precision, 273 tiles 1867 -> 1463 us,
+// 1093 (a grid of 2048) 2380 -> 1884, 3280 (a grid of 4096) 3015 -> 3655.
+constexpr int kAllTiles2D = 4096, kAllTiles3D = 2048;
+bool launch_all_orders(const BatchView& b) {
+  return b.tile == kAllTile && b.tile_cap <= (b.dim == 2 ? kAllTiles2D : kAllTiles3D);
+}
+
 template <typename T>
 void trace(const BatchView& b, const BatchTables& t, int in, int tr, hipStream_t s) {
+  if (launch_all_orders(b)) {
+    INSP_DIMT(hipLaunchKernelGGL((kb_trace_all<D_, T>), tiles_grid(b), dim3(kAllTile), 0, s, b, t, in, tr));
+    check("kb_trace_all");
+    return;
+  }
 #define INSP_TRACE(NN)                                                                              \
   INSP_DIMT(INSP_TB(hipLaunchKernelGGL((kb_trace<TB_, D_, T, NN>), dim3((unsigned)b.ocap[NN]), dim3(TB_), \
                                        0, s, b, t, in, tr)))
@@ -702,6 +763,9 @@ void apply(const BatchView& b, const BatchTables& t, int level, int in, int tr, 
   if (level) {
     INSP_DIMT(INSP_TB(hipLaunchKernelGGL((kb_apply<TB_, D_, T, 1, true>), tiles_grid(b), dim3(TB_), 0, s, b,
                                          t, in, tr, out, (int)dot)));
+  } else if (launch_all_orders(b)) {
+    INSP_DIMT(hipLaunchKernelGGL((kb_apply_all<D_, T>), tiles_grid(b), dim3(kAllTile), 0, s, b, t, in, tr, out,
+                                 (int)dot));
   } else {
 #define INSP_APPLY(NN)                                                                              \
   INSP_DIMT(INSP_TB(hipLaunchKernelGGL((kb_apply<TB_, D_, T, NN, false>), dim3((unsigned)b.ocap[NN]),      \
