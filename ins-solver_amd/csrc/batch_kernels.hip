@@ -65,6 +65,26 @@ __device__ __forceinline__ Cell locate(const BatchView& b) {
   return c;
 }
 
+// Vector passes walk a cell's rows in groups of kRows (the row counts 3, 6, 10, 15 and 4, 10, 20,
+// 35 leave at most two of a group idle): a group's loads are all issued before its first use. One
+// row at a time a pass over a few thousand tiles lasts as long as its chain of loads, one memory
+// latency per row. With the AMG products below one row to a group, a lockstep iteration of 2D problems of
+// orders 2-4 (mixed precision) went from 670 to 598 us at 1518 tiles and from 1595 to 1553 at 6075.
+constexpr int kRows = 5;
+
+template <typename T>
+__device__ __forceinline__ void load_rows(T (&v)[kRows], const T* x, int64_t S, int64_t e, int i0, int rows) {
+#pragma unroll
+  for (int k = 0; k < kRows; ++k) v[k] = x[(int64_t)min(i0 + k, rows - 1) * S + e];
+}
+
+template <typename T>
+__device__ __forceinline__ void store_rows(const T (&v)[kRows], T* x, int64_t S, int64_t e, int i0, int rows) {
+#pragma unroll
+  for (int k = 0; k < kRows; ++k)
+    if (i0 + k < rows) x[(int64_t)(i0 + k) * S + e] = v[k];
+}
+
 template <int TB, int K>
 __device__ __forceinline__ void put_partials(const BatchView& b, const Cell& c, const double (&v)[K]) {
   if (!c.live) return;  // uniform per block
@@ -223,10 +243,21 @@ kb_dot(BatchView b, int level, int fa, int fb, int fc, int fd, int nvals) {
     const T *a = (const T*)P.v[fa], *bb = (const T*)P.v[fb];
     const T *cc = nvals > 1 ? (const T*)P.v[fc] : nullptr, *dd = nvals > 1 ? (const T*)P.v[fd] : nullptr;
     const int rows = rows_of<T>(P, level);
-    for (int i = 0; i < rows; ++i) {
-      const int64_t q = i * P.S + c.e;
-      v[0] += (double)a[q] * (double)bb[q];
-      if (nvals > 1) v[1] += (double)cc[q] * (double)dd[q];
+    const int64_t S = P.S;
+    for (int i0 = 0; i0 < rows; i0 += kRows) {
+      T av[kRows], bv[kRows], cv[kRows], ev[kRows];
+      load_rows(av, a, S, c.e, i0, rows);
+      load_rows(bv, bb, S, c.e, i0, rows);
+      if (nvals > 1) {
+        load_rows(cv, cc, S, c.e, i0, rows);
+        load_rows(ev, dd, S, c.e, i0, rows);
+      }
+#pragma unroll
+      for (int k = 0; k < kRows; ++k) {
+        if (i0 + k >= rows) break;
+        v[0] += (double)av[k] * (double)bv[k];
+        if (nvals > 1) v[1] += (double)cv[k] * (double)ev[k];
+      }
     }
   }
   put_partials<TB, 2>(b, c, v);
@@ -243,13 +274,25 @@ __global__ void __launch_bounds__(TB) kb_fcg_update_xr(BatchView b) {
     const double alpha = sdiv(P.scal[BS_RZ], P.scal[BS_PAP]);
     double *x = (double*)P.v[BV_X], *r = (double*)P.v[BV_R];
     const double *p = (const double*)P.v[BV_P], *Ap = (const double*)P.v[BV_AP], *z = (const double*)P.v[BV_Z];
-    for (int i = 0; i < P.Np; ++i) {
-      const int64_t q = i * P.S + c.e;
-      x[q] = fma(alpha, p[q], x[q]);
-      const double ri = fma(-alpha, Ap[q], r[q]);
-      r[q] = ri;
-      v[0] += ri * ri;
-      v[1] += ri * z[q];
+    const int rows = P.Np;
+    const int64_t S = P.S;
+    for (int i0 = 0; i0 < rows; i0 += kRows) {
+      double xv[kRows], pv[kRows], rv[kRows], qv[kRows], zv[kRows];
+      load_rows(xv, x, S, c.e, i0, rows);
+      load_rows(pv, p, S, c.e, i0, rows);
+      load_rows(rv, r, S, c.e, i0, rows);
+      load_rows(qv, Ap, S, c.e, i0, rows);
+      load_rows(zv, z, S, c.e, i0, rows);
+#pragma unroll
+      for (int k = 0; k < kRows; ++k) {
+        if (i0 + k >= rows) break;
+        xv[k] = fma(alpha, pv[k], xv[k]);
+        rv[k] = fma(-alpha, qv[k], rv[k]);
+        v[0] += rv[k] * rv[k];
+        v[1] += rv[k] * zv[k];
+      }
+      store_rows(xv, x, S, c.e, i0, rows);
+      store_rows(rv, r, S, c.e, i0, rows);
     }
   }
   put_partials<TB, 2>(b, c, v);
@@ -264,9 +307,15 @@ __global__ void __launch_bounds__(TB) kb_fcg_update_p(BatchView b) {
   const double beta = sdiv(P.scal[BS_RZN] - P.scal[BS_RZO], P.scal[BS_RZ]);
   double* p = (double*)P.v[BV_P];
   const double* z = (const double*)P.v[BV_Z];
-  for (int i = 0; i < P.Np; ++i) {
-    const int64_t q = i * P.S + c.e;
-    p[q] = fma(beta, p[q], z[q]);
+  const int rows = P.Np;
+  const int64_t S = P.S;
+  for (int i0 = 0; i0 < rows; i0 += kRows) {
+    double pv[kRows], zv[kRows];
+    load_rows(pv, p, S, c.e, i0, rows);
+    load_rows(zv, z, S, c.e, i0, rows);
+#pragma unroll
+    for (int k = 0; k < kRows; ++k) pv[k] = fma(beta, pv[k], zv[k]);
+    store_rows(pv, p, S, c.e, i0, rows);
   }
 }
 
@@ -316,11 +365,19 @@ __global__ void __launch_bounds__(TB) kb_residual(BatchView b) {
     const BatchProb& P = b.P[c.slot];
     const double *bb = (const double*)P.v[BV_B], *Ap = (const double*)P.v[BV_AP];
     double* r = (double*)P.v[BV_R];
-    for (int i = 0; i < P.Np; ++i) {
-      const int64_t q = i * P.S + c.e;
-      const double t = bb[q] - Ap[q];
-      r[q] = t;
-      v[0] += t * t;
+    const int rows = P.Np;
+    const int64_t S = P.S;
+    for (int i0 = 0; i0 < rows; i0 += kRows) {
+      double bv[kRows], qv[kRows];
+      load_rows(bv, bb, S, c.e, i0, rows);
+      load_rows(qv, Ap, S, c.e, i0, rows);
+#pragma unroll
+      for (int k = 0; k < kRows; ++k) {
+        if (i0 + k >= rows) break;
+        bv[k] = bv[k] - qv[k];
+        v[0] += bv[k] * bv[k];
+      }
+      store_rows(bv, r, S, c.e, i0, rows);
     }
   }
   put_partials<TB, 1>(b, c, v);
@@ -333,7 +390,16 @@ __global__ void __launch_bounds__(TB) kb_convert(BatchView b, int src, int dst) 
   const BatchProb& P = b.P[c.slot];
   const Tin* x = (const Tin*)P.v[src];
   Tout* y = (Tout*)P.v[dst];
-  for (int i = 0; i < P.Np; ++i) y[i * P.S + c.e] = (Tout)x[i * P.S + c.e];
+  const int rows = P.Np;
+  const int64_t S = P.S;
+  for (int i0 = 0; i0 < rows; i0 += kRows) {
+    Tin xv[kRows];
+    Tout yv[kRows];
+    load_rows(xv, x, S, c.e, i0, rows);
+#pragma unroll
+    for (int k = 0; k < kRows; ++k) yv[k] = (Tout)xv[k];
+    store_rows(yv, y, S, c.e, i0, rows);
+  }
 }
 
 template <int TB, typename T>
@@ -347,12 +413,24 @@ __global__ void __launch_bounds__(TB) kb_cheb(BatchView b, int level, int step, 
   const T *f = (const T*)P.v[level ? BV_CB : BV_VB], *ax = (const T*)P.v[level ? BV_CAP : BV_VAX];
   T *d = (T*)P.v[level ? BV_CZ : BV_VD], *x = (T*)P.v[level ? BV_CX : BV_VX];
   const T c1 = (T)(level ? P.amg.oc1[step] : P.c1[step]), c2 = (T)(level ? P.amg.oc2[step] : P.c2[step]);
-  for (int i = 0; i < rows; ++i) {
-    const int64_t q = i * P.S + c.e;
-    const T res = inv[q] * (zero_init ? f[q] : f[q] - ax[q]);
-    const T di = step == 0 ? c2 * res : fma(c1, d[q], c2 * res);
-    d[q] = di;
-    x[q] = zero_init ? di : x[q] + di;
+  const int64_t S = P.S;
+  for (int i0 = 0; i0 < rows; i0 += kRows) {
+    T iv[kRows], fv[kRows], av[kRows], dv[kRows], xv[kRows];
+    load_rows(iv, inv, S, c.e, i0, rows);
+    load_rows(fv, f, S, c.e, i0, rows);
+    if (!zero_init) {
+      load_rows(av, ax, S, c.e, i0, rows);
+      load_rows(xv, x, S, c.e, i0, rows);
+    }
+    if (step) load_rows(dv, d, S, c.e, i0, rows);
+#pragma unroll
+    for (int k = 0; k < kRows; ++k) {
+      const T res = iv[k] * (zero_init ? fv[k] : fv[k] - av[k]);
+      dv[k] = step == 0 ? c2 * res : fma(c1, dv[k], c2 * res);
+      xv[k] = zero_init ? dv[k] : xv[k] + dv[k];
+    }
+    store_rows(dv, d, S, c.e, i0, rows);
+    store_rows(xv, x, S, c.e, i0, rows);
   }
 }
 
@@ -364,9 +442,14 @@ __global__ void __launch_bounds__(TB) kb_sub_from_b(BatchView b, int level) {
   const int rows = level ? P.Np1 : P.Np;
   const T* f = (const T*)P.v[level ? BV_CB : BV_VB];
   T* ax = (T*)P.v[level ? BV_CAP : BV_VAX];
-  for (int i = 0; i < rows; ++i) {
-    const int64_t q = i * P.S + c.e;
-    ax[q] = f[q] - ax[q];
+  const int64_t S = P.S;
+  for (int i0 = 0; i0 < rows; i0 += kRows) {
+    T fv[kRows], av[kRows];
+    load_rows(fv, f, S, c.e, i0, rows);
+    load_rows(av, ax, S, c.e, i0, rows);
+#pragma unroll
+    for (int k = 0; k < kRows; ++k) av[k] = fv[k] - av[k];
+    store_rows(av, ax, S, c.e, i0, rows);
   }
 }
 
@@ -420,8 +503,9 @@ __global__ void __launch_bounds__(TB) kb_vertex_prolong(BatchView b) {
 
 // CSR products over a 256-row tile of AMG level k: groups of kCsrLanes adjacent lanes share a
 // row (lane l takes the row's nonzeros l, l + kCsrLanes, ...) and add their partial sums by
-// shuffles in a fixed order; each group walks kCsrLanes rows of the tile. Returns the tile's
-// problem slot and first row, or slot -1 when the block has no live tile.
+// shuffles in a fixed order; block (x, y) of the grid takes a tile's rows of part y, one row to a
+// group, as one group's chain of pointer, index and value loads is what such a launch lasts.
+// Returns the tile's problem slot and first row, or slot -1 when the block has no live tile.
 constexpr int kCsrLanes = 8;
 __device__ __forceinline__ int2 locate_tile(const BatchView& b, int k) {
   const int t = (int)xcd_block();
@@ -454,12 +538,10 @@ __global__ void __launch_bounds__(kB) kb_amg_spmv(BatchView b, int k, int residu
   const T* x = (const T*)L.x;
   constexpr int G = kB / kCsrLanes;
   const int g = (int)threadIdx.x / kCsrLanes;
-  for (int i = 0; i < kCsrLanes; ++i) {
-    const int r = tt.y + g + G * i;
-    const bool live = r < L.n;
-    const T s = csr_row_dot<T>(L.Aptr, L.Acol, val, x, r, live);
-    if (live && threadIdx.x % kCsrLanes == 0) ((T*)L.r)[r] = residual ? ((const T*)L.b)[r] - s : s;
-  }
+  const int r = tt.y + g + G * (int)blockIdx.y;
+  const bool live = r < L.n;
+  const T s = csr_row_dot<T>(L.Aptr, L.Acol, val, x, r, live);
+  if (live && threadIdx.x % kCsrLanes == 0) ((T*)L.r)[r] = residual ? ((const T*)L.b)[r] - s : s;
 }
 
 template <typename T>
@@ -490,12 +572,10 @@ __global__ void __launch_bounds__(kB) kb_amg_restrict(BatchView b, int k) {
   const T* res = (const T*)L.r;
   constexpr int G = kB / kCsrLanes;
   const int g = (int)threadIdx.x / kCsrLanes;
-  for (int i = 0; i < kCsrLanes; ++i) {
-    const int r = tt.y + g + G * i;
-    const bool live = r < nc;
-    const T s = csr_row_dot<T>(L.Rptr, L.Rcol, val, res, r, live);
-    if (live && threadIdx.x % kCsrLanes == 0) ((T*)P.amg.lev[k + 1].b)[r] = s;
-  }
+  const int r = tt.y + g + G * (int)blockIdx.y;
+  const bool live = r < nc;
+  const T s = csr_row_dot<T>(L.Rptr, L.Rcol, val, res, r, live);
+  if (live && threadIdx.x % kCsrLanes == 0) ((T*)P.amg.lev[k + 1].b)[r] = s;
 }
 
 // Rows of level k: x_k += P_k x_{k+1}.
@@ -524,8 +604,21 @@ __global__ void __launch_bounds__(kB) kb_amg_dense(BatchView b, int k) {
   if (i >= n) return;
   const T* M = (const T*)P.amg.cinv;
   const T* bb = (const T*)P.amg.lev[k].b;
+  // 16 columns' loads in flight; the sum keeps its order
+  constexpr int C = 16;
   T s = 0;
-  for (int q = 0; q < n; ++q) s = fma(M[(int64_t)q * n + i], bb[q], s);
+  int q = 0;
+  for (; q + C <= n; q += C) {
+    T m[C], v[C];
+#pragma unroll
+    for (int c = 0; c < C; ++c) {
+      m[c] = M[(int64_t)(q + c) * n + i];
+      v[c] = bb[q + c];
+    }
+#pragma unroll
+    for (int c = 0; c < C; ++c) s = fma(m[c], v[c], s);
+  }
+  for (; q < n; ++q) s = fma(M[(int64_t)q * n + i], bb[q], s);
   ((T*)P.amg.lev[k].x)[i] = s;
 }
 
@@ -622,13 +715,26 @@ __global__ void __launch_bounds__(TB) kb_cg_xr(BatchView b, int num) {
     const T* inv = (const T*)P.invC[prec];
     const T *p = (const T*)P.v[BV_CP], *Ap = (const T*)P.v[BV_CAP];
     T *x = (T*)P.v[BV_CX], *r = (T*)P.v[BV_CR], *z = (T*)P.v[BV_CZ];
-    for (int i = 0; i < P.Np1; ++i) {
-      const int64_t q = i * P.S + c.e;
-      x[q] = fma(a, p[q], x[q]);
-      const T ri = fma(-a, Ap[q], r[q]), zi = inv[q] * ri;
-      r[q] = ri;
-      z[q] = zi;
-      v[0] += (double)ri * (double)zi;
+    const int rows = P.Np1;
+    const int64_t S = P.S;
+    for (int i0 = 0; i0 < rows; i0 += kRows) {
+      T xv[kRows], pv[kRows], rv[kRows], qv[kRows], zv[kRows];
+      load_rows(xv, x, S, c.e, i0, rows);
+      load_rows(pv, p, S, c.e, i0, rows);
+      load_rows(rv, r, S, c.e, i0, rows);
+      load_rows(qv, Ap, S, c.e, i0, rows);
+      load_rows(zv, inv, S, c.e, i0, rows);
+#pragma unroll
+      for (int k = 0; k < kRows; ++k) {
+        if (i0 + k >= rows) break;
+        xv[k] = fma(a, pv[k], xv[k]);
+        rv[k] = fma(-a, qv[k], rv[k]);
+        zv[k] = zv[k] * rv[k];
+        v[0] += (double)rv[k] * (double)zv[k];
+      }
+      store_rows(xv, x, S, c.e, i0, rows);
+      store_rows(rv, r, S, c.e, i0, rows);
+      store_rows(zv, z, S, c.e, i0, rows);
     }
   }
   put_partials<TB, 1>(b, c, v);
@@ -642,9 +748,15 @@ __global__ void __launch_bounds__(TB) kb_cg_p(BatchView b, int num, int den) {
   const T beta = (T)sdiv(P.scal[num], P.scal[den]);
   const T* z = (const T*)P.v[BV_CZ];
   T* p = (T*)P.v[BV_CP];
-  for (int i = 0; i < P.Np1; ++i) {
-    const int64_t q = i * P.S + c.e;
-    p[q] = fma(beta, p[q], z[q]);
+  const int rows = P.Np1;
+  const int64_t S = P.S;
+  for (int i0 = 0; i0 < rows; i0 += kRows) {
+    T pv[kRows], zv[kRows];
+    load_rows(pv, p, S, c.e, i0, rows);
+    load_rows(zv, z, S, c.e, i0, rows);
+#pragma unroll
+    for (int k = 0; k < kRows; ++k) pv[k] = fma(beta, pv[k], zv[k]);
+    store_rows(pv, p, S, c.e, i0, rows);
   }
 }
 
@@ -655,7 +767,15 @@ __global__ void __launch_bounds__(TB) kb_sum_d(BatchView b, int field) {
   if (c.valid) {
     const BatchProb& P = b.P[c.slot];
     const double* x = (const double*)P.v[field];
-    for (int i = 0; i < P.Np; ++i) v[0] += x[i * P.S + c.e];
+    const int rows = P.Np;
+    const int64_t S = P.S;
+    for (int i0 = 0; i0 < rows; i0 += kRows) {
+      double xv[kRows];
+      load_rows(xv, x, S, c.e, i0, rows);
+#pragma unroll
+      for (int k = 0; k < kRows; ++k)
+        if (i0 + k < rows) v[0] += xv[k];
+    }
   }
   put_partials<TB, 1>(b, c, v);
 }
@@ -668,7 +788,15 @@ __global__ void __launch_bounds__(TB) kb_sub_mean_d(BatchView b, int field) {
   if (!P.nullspace) return;
   const double m = P.scal[BS_MEAN] / P.dofs;
   double* x = (double*)P.v[field];
-  for (int i = 0; i < P.Np; ++i) x[i * P.S + c.e] -= m;
+  const int rows = P.Np;
+  const int64_t S = P.S;
+  for (int i0 = 0; i0 < rows; i0 += kRows) {
+    double xv[kRows];
+    load_rows(xv, x, S, c.e, i0, rows);
+#pragma unroll
+    for (int k = 0; k < kRows; ++k) xv[k] -= m;
+    store_rows(xv, x, S, c.e, i0, rows);
+  }
 }
 
 template <int TB>
@@ -697,7 +825,15 @@ __global__ void __launch_bounds__(TB) kb_inv_apply_d(BatchView b, int level, int
   const double* inv = (const double*)(level ? P.invC[0] : P.invF[0]);
   double* x = (double*)P.v[field];
   const int rows = level ? P.Np1 : P.Np;
-  for (int i = 0; i < rows; ++i) x[i * P.S + c.e] *= inv[i * P.S + c.e];
+  const int64_t S = P.S;
+  for (int i0 = 0; i0 < rows; i0 += kRows) {
+    double xv[kRows], iv[kRows];
+    load_rows(xv, x, S, c.e, i0, rows);
+    load_rows(iv, inv, S, c.e, i0, rows);
+#pragma unroll
+    for (int k = 0; k < kRows; ++k) xv[k] *= iv[k];
+    store_rows(xv, x, S, c.e, i0, rows);
+  }
 }
 
 template <int TB>
@@ -707,7 +843,15 @@ __global__ void __launch_bounds__(TB) kb_scale_d(BatchView b, int field, int slo
   const BatchProb& P = b.P[c.slot];
   const double s = P.scal[slot] > 0 ? 1.0 / sqrt(P.scal[slot]) : 0.0;
   double* x = (double*)P.v[field];
-  for (int i = 0; i < P.Np; ++i) x[i * P.S + c.e] *= s;
+  const int rows = P.Np;
+  const int64_t S = P.S;
+  for (int i0 = 0; i0 < rows; i0 += kRows) {
+    double xv[kRows];
+    load_rows(xv, x, S, c.e, i0, rows);
+#pragma unroll
+    for (int k = 0; k < kRows; ++k) xv[k] *= s;
+    store_rows(xv, x, S, c.e, i0, rows);
+  }
 }
 
 dim3 tiles_grid(const BatchView& b) { return dim3((unsigned)b.tile_cap); }
@@ -859,7 +1003,7 @@ void vertex_prolong(const BatchView& b, hipStream_t s) {
 
 template <typename T>
 void amg_spmv(const BatchView& b, int k, bool residual, hipStream_t s) {
-  hipLaunchKernelGGL((kb_amg_spmv<T>), dim3((unsigned)b.ltile_cap), dim3(kB), 0, s, b, k, (int)residual);
+  hipLaunchKernelGGL((kb_amg_spmv<T>), dim3((unsigned)b.ltile_cap, kCsrLanes), dim3(kB), 0, s, b, k, (int)residual);
   check("kb_amg_spmv");
 }
 
@@ -872,7 +1016,7 @@ void amg_cheb(const BatchView& b, int k, int step, bool zero_init, hipStream_t s
 
 template <typename T>
 void amg_restrict(const BatchView& b, int k, hipStream_t s) {
-  hipLaunchKernelGGL((kb_amg_restrict<T>), dim3((unsigned)b.ltile_cap), dim3(kB), 0, s, b, k);
+  hipLaunchKernelGGL((kb_amg_restrict<T>), dim3((unsigned)b.ltile_cap, kCsrLanes), dim3(kB), 0, s, b, k);
   check("kb_amg_restrict");
 }
 
