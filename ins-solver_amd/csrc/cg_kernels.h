@@ -8,6 +8,7 @@
 #include <cstdint>
 
 #include "kernels.h"
+#include "partials.h"
 
 namespace insp {
 
@@ -31,8 +32,6 @@ struct CgSlots {
 // from L2. 3D order-1 iteration: 236k cells 32.9 -> 29.1 us folded; 547k cells with 2136 partials read by
 // 2136 blocks 57.4 -> 58.5, by 1068 blocks 54.5.
 inline bool fold_pays(int64_t parts, int64_t blocks) { return parts * blocks <= 2400000; }
-// Blocks of the streams below on vectors of n entries.
-int cg_stream_blocks(int64_t n);
 
 // x = 0, z = p = inv b; partials of b.z. Returns their number. n is even, every vector 16-byte
 // aligned (as below).

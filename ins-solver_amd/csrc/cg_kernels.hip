@@ -18,7 +18,7 @@ inline void check(const char* what) {
     throw std::runtime_error(std::string("kernel launch failed: ") + what + ": " + hipGetErrorString(e));
 }
 
-constexpr int kBlock = 256;
+constexpr int kBlock = kPartBlock;
 
 // Sum of the partials, by the whole block; every thread gets it. Four loads in flight per thread,
 // added in an order that depends on n alone, so all blocks and all kernels form the same value.
@@ -256,34 +256,23 @@ k_p1_direction(int64_t E, int64_t stride, const T* __restrict__ z, const T* __re
   put_partial(dotv, partial);
 }
 
-// Pairs per thread of the streams: one, two or four while that leaves about a thousand blocks, whose
-// partials (and their reading of others') are cheap; longer vectors stream at two per thread and leave
-// the partials to a kernel in between. us per coarse iteration, 3D order 1: 547k cells with two per
-// thread and finalize 57.3, four and folded 54.5; 1.57M cells 157.4, eight and folded 161.1.
-int per_thread(int64_t n2) {
-  if (n2 <= (int64_t)kBlock * 1024) return 1;
-  if (n2 <= (int64_t)kBlock * 2 * 1024 || n2 > (int64_t)kBlock * 4 * 1536) return 2;
-  return 4;
-}
-int blocks(int64_t n2, int per) { return (int)((n2 + (int64_t)kBlock * per - 1) / ((int64_t)kBlock * per)); }
+int blocks(int64_t n2, int per) { return (int)cg_blocks(n2, per); }
 
 }  // namespace
 
 #define INSP_PER(n2, CALL)                       \
   do {                                           \
-    switch (per_thread(n2)) {                    \
+    switch (cg_pairs(n2)) {                      \
       case 1: { constexpr int P_ = 1; CALL; } break; \
       case 2: { constexpr int P_ = 2; CALL; } break; \
       default: { constexpr int P_ = 4; CALL; }   \
     }                                            \
   } while (0)
 
-int cg_stream_blocks(int64_t n) { return blocks(n / 2, per_thread(n / 2)); }
-
 template <typename T>
 int cg_init(int64_t n, const T* b, const T* inv, T* x, T* z, T* p, double* partial, hipStream_t s) {
   const int64_t n2 = n / 2;
-  const int nb = blocks(n2, per_thread(n2));
+  const int nb = blocks(n2, cg_pairs(n2));
   INSP_PER(n2, hipLaunchKernelGGL((k_cg_init<T, P_>), dim3(nb), dim3(kBlock), 0, s, n2, b, inv, x, z, p, partial));
   check("k_cg_init");
   return nb;
@@ -293,7 +282,7 @@ template <typename T>
 int cg_update_z(int64_t n, T* z, const T* Ap, const T* inv, Parts pap, const CgSlots& c, double* partial,
                 hipStream_t s) {
   const int64_t n2 = n / 2;
-  const int nb = blocks(n2, per_thread(n2));
+  const int nb = blocks(n2, cg_pairs(n2));
   INSP_PER(n2, hipLaunchKernelGGL((k_cg_z<T, P_>), dim3(nb), dim3(kBlock), 0, s, n2, z, Ap, inv, pap, c, partial));
   check("k_cg_z");
   return nb;
@@ -302,7 +291,7 @@ int cg_update_z(int64_t n, T* z, const T* Ap, const T* inv, Parts pap, const CgS
 template <typename T>
 void cg_update_p(int64_t n, T* p_next, const T* p, const T* z, Parts rz, const CgSlots& c, hipStream_t s) {
   const int64_t n2 = n / 2;
-  const int nb = blocks(n2, per_thread(n2));
+  const int nb = blocks(n2, cg_pairs(n2));
   INSP_PER(n2, hipLaunchKernelGGL((k_cg_p<T, P_>), dim3(nb), dim3(kBlock), 0, s, n2, p_next, p, z, rz, c));
   check("k_cg_p");
 }
@@ -311,7 +300,7 @@ template <typename T>
 void cg_update_x2p(int64_t n, T* x, T* p0, const T* p1, const T* z, Parts rz, const CgSlots& c, bool last,
                    hipStream_t s) {
   const int64_t n2 = n / 2;
-  const int nb = blocks(n2, per_thread(n2));
+  const int nb = blocks(n2, cg_pairs(n2));
   INSP_PER(n2, hipLaunchKernelGGL((k_cg_x2p<T, P_>), dim3(nb), dim3(kBlock), 0, s, n2, x, p0, p1, z, rz, c, last));
   check("k_cg_x2p");
 }

@@ -3,9 +3,9 @@
 
 #include <hip/hip_runtime.h>
 
-namespace insp {
+#include "partials.h"
 
-constexpr int kRedBlocks = 8192;  // partials per reduction slot (vector kernels)
+namespace insp {
 
 __device__ __forceinline__ double wave_sum(double v) {
 #pragma unroll

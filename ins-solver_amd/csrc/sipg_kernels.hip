@@ -485,7 +485,7 @@ template void launch_apply_p1_cells<double>(const MeshView&, const LevelView&, c
 template void launch_apply_p1_cells<float>(const MeshView&, const LevelView&, const float*,
                                            const float*, float*, hipStream_t, double*);
 
-int apply_blocks(int64_t E) { return (int)((E + 255) / 256); }
+int apply_blocks(int64_t E) { return (int)one_thread_blocks(E); }
 
 void launch_apply_slip(const MeshView& m, const LevelView& l, const double* u, const double* tr,
                        const double* kfac, double* out, const SlipFaces<double>& slip, hipStream_t s,

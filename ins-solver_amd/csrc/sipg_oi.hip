@@ -487,7 +487,7 @@ int launch_apply_oi(const MeshView& m, const LevelView& l, const OiView<T>& o, c
   if (m.E == 0) return 0;
   // four waves to a cell wherever the neighbour words are packed (meshes below 2^26 cells)
   if (m.nbc) {
-    const dim3 grid((unsigned)((m.E + 63) / 64));
+    const dim3 grid((unsigned)four_wave_blocks(m.E));
     INSP_OI_DISPATCH(m.dim, l.N,
                      hipLaunchKernelGGL((k_trace_oi_split<D_, N_, T>), grid, dim3(256), 0, s, m.E, m.stride, u,
                                         m.Kt, o.ks, o.C, o.tU, o.tT));

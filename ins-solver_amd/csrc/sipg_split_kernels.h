@@ -21,7 +21,7 @@ inline void check(const char* what) {
 }
 
 constexpr int kCells = 64;  // cells of a block
-inline dim3 grid_split(int64_t E) { return dim3((unsigned)((E + kCells - 1) / kCells)); }
+inline dim3 grid_split(int64_t E) { return dim3((unsigned)four_wave_blocks(E)); }
 
 template <int DIM, int N, typename T, bool VAR>
 __global__ void __launch_bounds__(256)

@@ -154,7 +154,7 @@ PoissonSolver::PoissonSolver(HostMesh mesh, int order, hipStream_t stream)
   bctype_.upload(bt.data(), bt.size());
   scal_.alloc(S_COUNT + P_COUNT);
   // two halves: the coarse CG leaves two sums as partials at a time
-  partial_.alloc((size_t)2 * std::max<int64_t>(4 * kRedBlocks, split_blocks(E)));
+  partial_.alloc((size_t)2 * partials_half(E, (int64_t)np() * stride_));
   INSP_HIP(hipHostMalloc((void**)&host_scal_, (S_COUNT + 2 * P_COUNT) * sizeof(double), hipHostMallocDefault));
   for (hipEvent_t& e : ev_pcg_) INSP_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
 }
@@ -922,7 +922,9 @@ void PoissonSolver::coarse_cg(int l) {
   // are too many for that, as one value added up by a kernel in between.
   double* const part_pap = partial_.p;
   double* const part_rz = partial_.p + partial_.n / 2;
-  const int consumer = cg_stream_blocks(n);
+  const int64_t consumer = cg_stream_blocks(n);
+  if ((size_t)std::max<int64_t>(consumer, split_blocks(mesh_.n_cells)) > partial_.n / 2)
+    throw std::logic_error("coarse CG: more partial sums than room for them");
   auto folded = [&](int np, double* part, int slot) {
     if (fold_pays(np, consumer)) return Parts{part, np};
     finalize(np, 1, part, scal_.p, slot, stream_);

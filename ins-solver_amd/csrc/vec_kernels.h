@@ -14,7 +14,7 @@
 namespace insp {
 
 struct RedScratch {
-  double* partial;  // max(kRedBlocks, apply blocks) * 4 doubles
+  double* partial;  // 4 * kRedBlocks doubles
 };
 
 int red_blocks(int64_t n);
