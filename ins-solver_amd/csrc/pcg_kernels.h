@@ -13,29 +13,25 @@
 #include <string>
 
 #include "cg_kernels.h"
+#include "pcg_state.h"
 #include "vec_kernels.h"
 
 namespace insp {
 
-// Device state of a run: r.z of this and of the next iteration (they trade places), p.Ap and |r|^2 of
-// the last one, the iterations done, why it stopped, and sums added by a kernel of their own.
-enum PcgSlot { P_RZ0 = 0, P_RZ1 = 1, P_PAP = 2, P_RR = 3, P_IT = 4, P_STOP = 5, P_SUM = 8, P_COUNT = 12 };
-enum PcgStop { PCG_RUNNING = 0, PCG_TOL = 1, PCG_BREAKDOWN = 2 };
-
 void pcg_start(double* st, hipStream_t s);  // running, no iterations done
-// x += a p, r -= a Ap, z = inv r with a = st[rz] / p.Ap; partials of |r|^2, r.z and r.(z - z_old), as many
+// x += a p, r -= a Ap, z = inv r with a = r.z / p.Ap; partials of |r|^2, r.z and r.(z - z_old), as many
 // as it returns of each, one after the other.
 int pcg_update_jacobi(int64_t n, double* x, double* r, double* z, const double* p, const double* Ap,
-                      const double* inv, Parts pap, double* st, int rz, double* partial, hipStream_t s);
+                      const double* inv, Parts pap, double* st, const PcgTurn& t, double* partial, hipStream_t s);
 // The same with z = scale (J M)^-1 r, or ((J M)^-1 r)_i / recp_i, on ncomp vectors cs apart.
 int pcg_update_inv_mass(int np, int ncomp, int64_t E, int64_t stride, int64_t cs, double* x, double* r,
                         double* z, const double* p, const double* Ap, const double* J, const double* Minv,
-                        double scale, const double* recp, Parts pap, double* st, int rz, double* partial,
+                        double scale, const double* recp, Parts pap, double* st, const PcgTurn& t, double* partial,
                         hipStream_t s);
 // Counts the iteration and stops it at |r| <= tol or on a breakdown, else p = z + beta p, from the nb
 // partials of each of the step's sums.
-void pcg_direction(int64_t n, double* p, const double* z, int nb, const double* partial, double* st, int rz_old,
-                   int rz_new, double tol, hipStream_t s);
+void pcg_direction(int64_t n, double* p, const double* z, int nb, const double* partial, double* st,
+                   const PcgTurn& t, double tol, hipStream_t s);
 
 // Entries up to which iterations are launched ahead: about 100 us each there (2D order 3, 2048 cells: 20
 // us, and as much again to wake the host and refill the queue after each look).
@@ -72,7 +68,7 @@ PcgEnd pcg_drive(int limit, bool ahead, const double* st, double* host, hipEvent
     ok(hipEventSynchronize(ev[head]));
     const double* h = host + head * P_COUNT;
     end.iterations = (int)h[P_IT];
-    end.stop = (int)h[P_STOP];
+    end.stop = pcg_stopped(h);
     end.rr = h[P_RR];
     head ^= 1;
     --out;

@@ -92,18 +92,18 @@ __global__ void __launch_bounds__(kBlock) k_pcg_sums(PcgSums sums, double* __res
 __global__ void k_pcg_start(double* st) {
   if (threadIdx.x == 0) {
     st[P_IT] = 0.0;
-    st[P_STOP] = (double)PCG_RUNNING;
+    st[P_STOP0] = st[P_STOP1] = (double)PCG_RUNNING;
   }
 }
 
 // Length of the step; the first block keeps p.Ap for the direction pass. False once stopped (the same
-// for every block: only the direction pass stops).
-__device__ __forceinline__ bool step_length(const Parts& pap, double* st, int rz, bool first, double* a) {
-  if (st[P_STOP] != (double)PCG_RUNNING) return false;
+// for every wave: only the direction pass stops).
+__device__ __forceinline__ bool step_length(const Parts& pap, double* st, const PcgTurn& t, bool first, double* a) {
+  if (!pcg_running(st, t)) return false;
   double v[1];
   totals<1>(pap.p, pap.n, 0, v);
   if (first && threadIdx.x == 0) st[P_PAP] = v[0];
-  *a = safe_div(st[rz], v[0]);
+  *a = safe_div(st[t.rz], v[0]);
   return true;
 }
 
@@ -112,9 +112,9 @@ __device__ __forceinline__ bool step_length(const Parts& pap, double* st, int rz
 __global__ void __launch_bounds__(kBlock)
 k_pcg_jacobi(int64_t n2, double2* __restrict__ x, double2* __restrict__ r, double2* __restrict__ z,
              const double2* __restrict__ p, const double2* __restrict__ Ap, const double2* __restrict__ inv,
-             Parts pap, double* st, int rz, double* __restrict__ partial) {
+             Parts pap, double* st, PcgTurn t, double* __restrict__ partial) {
   double a;
-  if (!step_length(pap, st, rz, blockIdx.x == 0, &a)) return;
+  if (!step_length(pap, st, t, blockIdx.x == 0, &a)) return;
   double v[3] = {0.0, 0.0, 0.0};
   auto one = [&](double& xi, double& ri, double& zi, double pi, double api, double di) {
     xi = fma(a, pi, xi);
@@ -144,10 +144,10 @@ __global__ void __launch_bounds__(kBlock)
 k_pcg_inv_mass(int64_t E, int64_t stride, int64_t cs, double* __restrict__ x, double* __restrict__ r,
                double* __restrict__ z, const double* __restrict__ p, const double* __restrict__ Ap,
                const double* __restrict__ J, const double* __restrict__ Minv, double scale,
-               const double* __restrict__ recp, Parts pap, double* st, int rz, double* __restrict__ partial) {
+               const double* __restrict__ recp, Parts pap, double* st, PcgTurn t, double* __restrict__ partial) {
   double a;
   const int64_t block = blockIdx.y * (int64_t)gridDim.x + blockIdx.x;
-  if (!step_length(pap, st, rz, block == 0, &a)) return;
+  if (!step_length(pap, st, t, block == 0, &a)) return;
   const cptr<double> Mi = as_const(Minv);
   const int64_t c0 = blockIdx.y * cs;
   double v[3] = {0.0, 0.0, 0.0};
@@ -180,24 +180,22 @@ k_pcg_inv_mass(int64_t E, int64_t stride, int64_t cs, double* __restrict__ x, do
   put3(v, block, (int64_t)gridDim.x * gridDim.y, partial);
 }
 
-// Every block forms the same sums and takes the same decision; the first one writes it down. A block
-// that reads the new P_STOP already returns as it would have by its own sums.
+// Every block forms the same sums and takes the same decision; the first one writes it down, into slots
+// that no wave of this launch reads (PcgTurn): all waves of a block go the same way to its barriers.
 __global__ void __launch_bounds__(kBlock)
 k_pcg_direction(int64_t n2, double2* __restrict__ p, const double2* __restrict__ z, PcgSums sums, double* st,
-                int rz_old, int rz_new, double tol) {
-  if (st[P_STOP] != (double)PCG_RUNNING) return;
-  const double ro = st[rz_old], pap = st[P_PAP];
+                PcgTurn t, double tol) {
+  const bool first = blockIdx.x == 0 && threadIdx.x == 0;
+  if (!pcg_running(st, t)) {
+    if (first) pcg_keep_stop(st, t);
+    return;
+  }
+  const double ro = st[t.rz], pap = st[P_PAP];
   double v[3];
   totals<3>(sums.p, sums.n, sums.stride, v);
-  const bool bad = !(pap > 0.0) || !isfinite(v[0]) || !isfinite(pap);
-  const bool met = !bad && sqrt(v[0]) <= tol;
-  if (blockIdx.x == 0 && threadIdx.x == 0) {
-    st[P_IT] += 1.0;
-    st[P_RR] = v[0];
-    st[rz_new] = v[1];
-    if (bad || met) st[P_STOP] = (double)(bad ? PCG_BREAKDOWN : PCG_TOL);
-  }
-  if (bad || met) return;
+  const PcgStop why = pcg_decide(v[0], pap, tol);
+  if (first) pcg_record(st, t, v[0], v[1], why);
+  if (why != PCG_RUNNING) return;
   const double beta = safe_div(v[2], ro);
   const int64_t i = blockIdx.x * (int64_t)kBlock + threadIdx.x;
   if (i >= n2) return;
@@ -223,25 +221,25 @@ void pcg_start(double* st, hipStream_t s) {
 }
 
 int pcg_update_jacobi(int64_t n, double* x, double* r, double* z, const double* p, const double* Ap,
-                      const double* inv, Parts pap, double* st, int rz, double* partial, hipStream_t s) {
+                      const double* inv, Parts pap, double* st, const PcgTurn& t, double* partial, hipStream_t s) {
   const int nb = stream_blocks(n / 2);
   auto v2 = [](const double* q) { return reinterpret_cast<const double2*>(q); };
   hipLaunchKernelGGL(k_pcg_jacobi, dim3(nb), dim3(kBlock), 0, s, n / 2, reinterpret_cast<double2*>(x),
                      reinterpret_cast<double2*>(r), reinterpret_cast<double2*>(z), v2(p), v2(Ap), v2(inv), pap,
-                     st, rz, partial);
+                     st, t, partial);
   check("k_pcg_jacobi");
   return nb;
 }
 
 int pcg_update_inv_mass(int np, int ncomp, int64_t E, int64_t stride, int64_t cs, double* x, double* r,
                         double* z, const double* p, const double* Ap, const double* J, const double* Minv,
-                        double scale, const double* recp, Parts pap, double* st, int rz, double* partial,
+                        double scale, const double* recp, Parts pap, double* st, const PcgTurn& t, double* partial,
                         hipStream_t s) {
   const dim3 grid((unsigned)((E + kBlock - 1) / kBlock), (unsigned)ncomp);
 #define INSP_IM(NP)                                                                                         \
   case NP:                                                                                                  \
     hipLaunchKernelGGL((k_pcg_inv_mass<NP>), grid, dim3(kBlock), 0, s, E, stride, cs, x, r, z, p, Ap, J, Minv, \
-                       scale, recp, pap, st, rz, partial);                                                  \
+                       scale, recp, pap, st, t, partial);                                                   \
     break
   switch (np) {
     INSP_IM(3);
@@ -258,8 +256,8 @@ int pcg_update_inv_mass(int np, int ncomp, int64_t E, int64_t stride, int64_t cs
   return (int)(grid.x * grid.y);
 }
 
-void pcg_direction(int64_t n, double* p, const double* z, int nb, const double* partial, double* st, int rz_old,
-                   int rz_new, double tol, hipStream_t s) {
+void pcg_direction(int64_t n, double* p, const double* z, int nb, const double* partial, double* st,
+                   const PcgTurn& t, double tol, hipStream_t s) {
   PcgSums sums{partial, nb, nb};
   if (nb > kFoldParts) {
     hipLaunchKernelGGL(k_pcg_sums, dim3(1), dim3(kBlock), 0, s, sums, st + P_SUM);
@@ -268,8 +266,7 @@ void pcg_direction(int64_t n, double* p, const double* z, int nb, const double* 
   }
   const int64_t n2 = n / 2;
   hipLaunchKernelGGL(k_pcg_direction, dim3((unsigned)((n2 + kBlock - 1) / kBlock)), dim3(kBlock), 0, s, n2,
-                     reinterpret_cast<double2*>(p), reinterpret_cast<const double2*>(z), sums, st, rz_old,
-                     rz_new, tol);
+                     reinterpret_cast<double2*>(p), reinterpret_cast<const double2*>(z), sums, st, t, tol);
   check("k_pcg_direction");
 }
 

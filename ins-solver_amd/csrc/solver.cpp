@@ -1444,20 +1444,20 @@ PcgEnd PoissonSolver::pcg_iterate(double tol, int limit) {
   double* const part_step = partial_.p + partial_.n / 2;
   pcg_start(st, stream_);
   auto step = [&](int k) {
-    const int rz = P_RZ0 + k % 2, rz_next = P_RZ0 + (k + 1) % 2;
+    const PcgTurn turn = pcg_turn(k);
     Parts pap{part_pap, apply_level<double>(0, p_.p, Ap_.p, part_pap)};  // p.Ap fused into the element pass
     if (pap.n > kFoldParts) {
       finalize(pap.n, 1, part_pap, st, P_SUM, stream_);
       pap = Parts{st + P_SUM, 1};
     }
     const int nb = type_ == SolverType::JACOBI_PCG
-                       ? pcg_update_jacobi(n, x_.p, r_.p, z_.p, p_.p, Ap_.p, levels_[0]->w64.inv.p, pap, st, rz,
+                       ? pcg_update_jacobi(n, x_.p, r_.p, z_.p, p_.p, Ap_.p, levels_[0]->w64.inv.p, pap, st, turn,
                                            part_step, stream_)
                        : pcg_update_inv_mass(np(), 1, mesh_.n_cells, stride_, 0, x_.p, r_.p, z_.p, p_.p, Ap_.p,
                                              J_.p, minv_.p, inv_mass_factor_,
-                                             inv_mass_recp_.empty() ? nullptr : inv_mass_recp_.p, pap, st, rz,
+                                             inv_mass_recp_.empty() ? nullptr : inv_mass_recp_.p, pap, st, turn,
                                              part_step, stream_);
-    pcg_direction(n, p_.p, z_.p, nb, part_step, st, rz, rz_next, tol, stream_);
+    pcg_direction(n, p_.p, z_.p, nb, part_step, st, turn, tol, stream_);
   };
   return pcg_drive(limit, n <= kAheadEntries, st, host_scal_ + S_COUNT, ev_pcg_, stream_, step);
 }

@@ -348,17 +348,17 @@ PcgEnd VecViscousSolver::pcg_iterate(double tol, int limit) {
   const double* recp = prec_ == VecPrecond::RECP_FACTOR_DAT_INV_MASS ? base_.inv_mass_recp_.p : nullptr;
   pcg_start(st, s);
   auto step = [&](int k) {
-    const int rz = P_RZ0 + k % 2, rz_next = P_RZ0 + (k + 1) % 2;
+    const PcgTurn turn = pcg_turn(k);
     Parts pap{part_pap, apply(p_.p, Ap_.p, part_pap)};
     if (pap.n > kFoldParts) {
       finalize(pap.n, 1, part_pap, st, P_SUM, s);
       pap = Parts{st + P_SUM, 1};
     }
     const int nb = prec_ == VecPrecond::JACOBI
-                       ? pcg_update_jacobi(n, x_.p, r_.p, z_.p, p_.p, Ap_.p, inv_.p, pap, st, rz, part_step, s)
+                       ? pcg_update_jacobi(n, x_.p, r_.p, z_.p, p_.p, Ap_.p, inv_.p, pap, st, turn, part_step, s)
                        : pcg_update_inv_mass(Np, ncomp_, E, stride, cs, x_.p, r_.p, z_.p, p_.p, Ap_.p, base_.J_.p,
-                                             minv_.p, scale, recp, pap, st, rz, part_step, s);
-    pcg_direction(n, p_.p, z_.p, nb, part_step, st, rz, rz_next, tol, s);
+                                             minv_.p, scale, recp, pap, st, turn, part_step, s);
+    pcg_direction(n, p_.p, z_.p, nb, part_step, st, turn, tol, s);
   };
   return pcg_drive(limit, n <= kAheadEntries, st, host_scal_ + V_COUNT, base_.ev_pcg_, s, step);
 }
