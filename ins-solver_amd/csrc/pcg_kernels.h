@@ -33,8 +33,7 @@ int pcg_update_inv_mass(int np, int ncomp, int64_t E, int64_t stride, int64_t cs
 void pcg_direction(int64_t n, double* p, const double* z, int nb, const double* partial, double* st,
                    const PcgTurn& t, double tol, hipStream_t s);
 
-// Entries up to which iterations are launched ahead: about 100 us each there (2D order 3, 2048 cells: 20
-// us, and as much again to wake the host and refill the queue after each look).
+// Entries up to which iterations are launched ahead: up to about 100 us each (2D order 3, 2048 cells: 20 us).
 constexpr int64_t kAheadEntries = int64_t(1) << 20;
 
 struct PcgEnd {
@@ -42,9 +41,9 @@ struct PcgEnd {
   double rr = 0;
 };
 
-// Launches iterations (step(k)) until one stops the run or `limit` are done. On short iterations
-// (`ahead`) eight at a time, the state of one eight looked at while the next runs: at most 15 are
-// launched in vain; otherwise one by one, each with its look.
+// Launches iterations (step(k)) until one stops the run or `limit` are done: on short iterations (`ahead`)
+// several to a look at the state and the next ones before it (pcg_batch, pcg_looks), otherwise one by
+// one, each with its look.
 template <class Step>
 PcgEnd pcg_drive(int limit, bool ahead, const double* st, double* host, hipEvent_t (&ev)[2], hipStream_t s,
                  Step&& step) {
@@ -54,8 +53,8 @@ PcgEnd pcg_drive(int limit, bool ahead, const double* st, double* host, hipEvent
   PcgEnd end;
   int done = 0, out = 0, head = 0, tail = 0;
   for (;;) {
-    if (done < limit && out < (ahead ? 2 : 1)) {
-      const int m = std::min(ahead ? 8 : 1, limit - done);
+    if (done < limit && out < (ahead ? pcg_looks(done) : 1)) {
+      const int m = std::min(ahead ? pcg_batch(done) : 1, limit - done);
       for (int k = 0; k < m; ++k) step(done + k);
       done += m;
       ok(hipMemcpyAsync(host + tail * P_COUNT, st, P_COUNT * sizeof(double), hipMemcpyDeviceToHost, s));

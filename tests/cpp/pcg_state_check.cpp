@@ -1,6 +1,7 @@
 // The state of a fused conjugate gradient run (pcg_state.h) under the orders in which a launch's waves may
 // come to it: a wave reads the state before and after the first block's thread has written it, and
-// must see the same; a run of iterations with several launched after its end.
+// must see the same; a run of iterations with several launched after its end; and how many a run that ends
+// after any number of iterations launches in vain.
 #include "pcg_state.h"
 
 #include <cstdio>
@@ -44,6 +45,20 @@ int main() {
         expect(st[P_RR] == 50.0 + (k + 1 < end ? k : end - 1), "|r|^2 of the last one", k);
       }
     }
+  for (int end = 1; end <= 2000; ++end) {
+    int done = 0, seen = 0, open[2] = {0, 0}, out = 0;  // iterations launched, looked at, and in each open look
+    while (seen < end) {
+      if (out < pcg_looks(done)) {
+        expect(out < 2, "open looks", end);
+        done += open[out++] = pcg_batch(done);
+      } else {
+        seen += open[0];
+        open[0] = open[1];
+        --out;
+      }
+    }
+    expect(done - end <= (end <= 3 ? 0 : 2 + end / 4) && done - end <= 15, "launched in vain", end);
+  }
   std::printf(bad ? "%d failures\n" : "ok\n", bad);
   return bad != 0;
 }

@@ -1,5 +1,5 @@
 """The fused CG's device state: no wave of a launch reads what another wave of it writes, and launches after
-the end change nothing (tests/cpp/pcg_state_check.cpp on the functions of ins-solver_amd/csrc/pcg_state.h
+the end change nothing and stay a small part of the run (tests/cpp/pcg_state_check.cpp on the functions of ins-solver_amd/csrc/pcg_state.h
 that the kernels call)."""
 import os
 import subprocess
