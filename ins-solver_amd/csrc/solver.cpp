@@ -6,6 +6,7 @@
 #include <cmath>
 #include <cstring>
 
+#include "caller_memory.h"
 #include "cg_kernels.h"
 #include "pcg_kernels.h"
 #include "split_passes.h"
@@ -31,6 +32,23 @@ bool disjoint(const double* a, const double* b, size_t n) {
   return x + n * sizeof(double) <= y || y + n * sizeof(double) <= x;
 }
 }  // namespace
+
+bool in_place(const double* p, size_t n) {
+  hipPointerAttribute_t a{};
+  void* base = nullptr;
+  CallerMemory m;
+  int gpu = -1;
+  if (hipGetDevice(&gpu) != hipSuccess || hipPointerGetAttributes(&a, p) != hipSuccess ||
+      hipMemGetAddressRange(reinterpret_cast<hipDeviceptr_t*>(&base), &m.size, const_cast<double*>(p)) !=
+          hipSuccess) {
+    (void)hipGetLastError();  // not an error of this call: the copies find their own
+    return false;
+  }
+  m.device = a.type == hipMemoryTypeDevice && !a.isManaged;
+  m.gpu = a.device;
+  m.base = reinterpret_cast<uintptr_t>(base);
+  return in_place(m, gpu, reinterpret_cast<uintptr_t>(p), n * sizeof(double));
+}
 
 template <typename T>
 struct PoissonSolver::Work {
@@ -350,11 +368,11 @@ void PoissonSolver::grad_central(const double* p, double* const g[3], const doub
   }
   const size_t n = (size_t)Np * stride_;
   const Level& l0 = *levels_[0];
-  // The caller's own vectors where they have the solver's layout and no output overlaps an input
+  // The caller's own vectors where they have the solver's layout, lie on this GPU and no output overlaps an input
   // that other threads still read: an output may be its own uT component, entry by entry.
-  bool direct = layout == Layout::DEVICE_SOA && dat_stride() == stride_;
+  bool direct = layout == Layout::DEVICE_SOA && dat_stride() == stride_ && in_place(p, n);
   for (int x = 0; x < d && direct; ++x) {
-    direct = disjoint(g[x], p, n);
+    direct = disjoint(g[x], p, n) && in_place(g[x], n) && !(u && u[x] && !in_place(u[x], n));
     for (int y = 0; y < d; ++y) {
       if (y != x) direct = direct && disjoint(g[x], g[y], n);
       if (u && u[y] && !(y == x && u[y] == g[x])) direct = direct && disjoint(g[x], u[y], n);
@@ -1559,7 +1577,8 @@ void PoissonSolver::mult(const double* in, double* out, Layout layout, bool fp32
   const int64_t E = mesh_.n_cells;
   // The caller's own vectors where they have the solver's layout: the passes read cells only, so
   // the input's padding may hold anything; the output's is cleared.
-  const bool own = layout == Layout::DEVICE_SOA && dat_stride() == stride_ && in && out;
+  const bool own = layout == Layout::DEVICE_SOA && dat_stride() == stride_ && in && out && in_place(in, n) &&
+                   in_place(out, n);
   if (!fp32) {
     if (own && disjoint(in, out, n)) {
       apply_level<double>(0, in, out);

@@ -85,3 +85,22 @@ def test_projection_on_the_callers_vectors(ip, dim, N):
     ud = [dev(v) for v in u]
     call(pd, ud, [pd] + od[1:])  # an output over the pressure
     _same(pd, want[0])
+
+
+@pytest.mark.parametrize("fp32", [False, True])
+def test_pinned_host_vectors_go_through_the_copies(ip, fp32):
+    """Memory that is not the GPU's own is copied, as every vector once was, with the same results."""
+    s = _solver(ip, 3, 2)
+    x = np.random.default_rng(7).standard_normal((s.n_cells, s.Np))
+    fn = s.mult_fp32 if fp32 else s.mult
+    want = fn(x)
+    pinned = torch.empty((s.Np, s.stride), dtype=torch.float64, pin_memory=True)
+    dev = _device(x, s.stride)
+    pinned.copy_(dev)
+    torch.cuda.synchronize()
+    out = torch.full_like(dev, float("nan"))
+    torch.cuda.synchronize()
+    fn((pinned.data_ptr(), out.data_ptr()), layout=ip.LAYOUT_DEVICE_SOA)
+    _same(out, want)
+    fn((dev.data_ptr(), pinned.data_ptr()), layout=ip.LAYOUT_DEVICE_SOA)
+    _same(pinned, want)
