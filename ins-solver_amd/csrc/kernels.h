@@ -74,7 +74,8 @@ void launch_trace(const MeshView& m, const LevelView& l, const T* u, const T* kf
 template <typename T>
 void launch_apply(const MeshView& m, const LevelView& l, const T* u, const T* tr, const T* kfac,
                   T* out, hipStream_t s, double* partial = nullptr);
-// The same with the mass term added by the element pass (orders >= 2, packed words, FP64).
+// The same with the mass term added by the element pass (orders >= 2 but 3D order 4, packed words, FP64).
+bool apply_mass_pays(const MeshView& m, const LevelView& l);
 void launch_apply_mass(const MeshView& m, const LevelView& l, const double* u, const double* tr,
                        const double* kfac, const MassView<double>& mass, double* out, hipStream_t s,
                        double* partial);

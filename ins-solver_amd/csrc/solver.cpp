@@ -782,7 +782,7 @@ int PoissonSolver::apply_level(int l, const T* u, T* out, double* partial, T* tr
     trace_pass<T>(mv, v, u, k, tr, stream_);
     if (prof) INSP_HIP(hipEventRecord(e1, stream_));
     if constexpr (std::is_same<T, double>::value) {
-      if (has_mass_term() && mv.nbc && lv.N >= 2) {
+      if (has_mass_term() && apply_mass_pays(mv, v)) {
         launch_apply_mass(mv, v, u, tr, k, MassView<double>{var_mm_ ? w.mm.p : nullptr, mm_const_}, out,
                           stream_, partial);
         mass_done = true;
