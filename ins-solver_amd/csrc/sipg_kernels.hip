@@ -52,8 +52,11 @@ k_trace(int64_t E, int64_t stride, const T* __restrict__ u, const double* __rest
   if (e < E) trace_cell<DIM, N, T, VAR>(e, stride, u, Kt, kfac, as_const(C), tr);
 }
 
+// Element pass. FP32 at 3D order 3 (and its Chebyshev form below) is held to the 128 registers of four waves
+// per SIMD; left alone it takes 132 to 138 and three waves: 584,016 cells with a coefficient 142 -> 127 us,
+// Chebyshev step 179 -> 158 us (five registers spilled there, none with k = 1).
 template <int DIM, int N, typename T, bool VAR, bool PACK>
-__global__ void __launch_bounds__(256)
+__global__ void __launch_bounds__(256, DIM == 3 && N == 3 && sizeof(T) == 4 ? 4 : 1)
 k_apply(int64_t E, int64_t stride, const T* __restrict__ u, const T* __restrict__ tr,
         const double* __restrict__ Kt, const double* __restrict__ tauS,
         const int* __restrict__ nbr, const int* __restrict__ code,
@@ -93,7 +96,7 @@ k_apply_p1(int64_t E, int64_t stride, const T* __restrict__ u, const double* __r
 
 // Element pass with the Chebyshev step of the smoother fused into its output (orders >= 2).
 template <int DIM, int N, typename T, bool VAR, bool PACK>
-__global__ void __launch_bounds__(256)
+__global__ void __launch_bounds__(256, DIM == 3 && N == 3 && sizeof(T) == 4 ? 4 : 1)
 k_apply_cheb(int64_t E, int64_t stride, const T* __restrict__ u, const T* __restrict__ tr,
              const double* __restrict__ Kt, const double* __restrict__ tauS,
              const int* __restrict__ nbr, const int* __restrict__ code,
@@ -124,9 +127,11 @@ k_apply_p1_cheb(int64_t E, int64_t stride, const T* __restrict__ u, const double
 }
 
 // Element pass of one component of the vector (velocity) operator with slip faces (FP64;
-// orders >= 2 read the face traces, order 1 recomputes them). kfac may be null (k = 1).
+// orders >= 2 read the face traces, order 1 recomputes them). kfac may be null (k = 1). 3D orders 2
+// and 3 are held to the 168 registers of three waves per SIMD, which they miss by one otherwise (no
+// spills; order 2, 511,104 cells, three components with their traces and mass terms 657 -> 620 us).
 template <int DIM, int N>
-__global__ void __launch_bounds__(256)
+__global__ void __launch_bounds__(256, DIM == 3 && (N == 2 || N == 3) ? 3 : 1)
 k_apply_slip(int64_t E, int64_t stride, const double* __restrict__ u, const double* __restrict__ tr,
              const double* __restrict__ Kt, const double* __restrict__ tauS,
              const int* __restrict__ nbr, const int* __restrict__ code,
