@@ -8,11 +8,13 @@ import pytest
 
 pytestmark = pytest.mark.gpu
 
-# (dim, order, hexes or squares per edge): 1 cell pair / 6 cells, remainders of 64 cells, and the
-# last mesh below and the first above 2^16, 1.5 x 2^16 and 3 x 2^16 cells
+# (dim, order, hexes or squares per edge): 1 cell pair / 6 cells, remainders of 64 cells, and meshes on both
+# sides of the lines of the element pass (2D 2^16 cells, order 4 3 x 2^16; 3D order 2 12 x 2^16, order 3 1.5
+# x 2^16 and FP32 2 x 2^16, order 4 2^16 and FP32 1.5 x 2^16) and of the trace pass (2D order 4 and 3D
+# order 2 3 x 2^16, 3D order 3 6 x 2^16)
 SIZES = [(2, 2, 1), (2, 3, 7), (2, 4, 23), (2, 2, 181), (2, 2, 182), (2, 3, 182), (2, 4, 313), (2, 4, 314),
          (3, 2, 1), (3, 3, 1), (3, 4, 2), (3, 3, 5), (3, 2, 31), (3, 2, 33), (3, 3, 25), (3, 3, 26), (3, 4, 22),
-         (3, 4, 23)]
+         (3, 4, 23), (3, 2, 50), (3, 2, 51), (3, 3, 28), (3, 3, 29), (3, 4, 25), (3, 4, 26), (3, 3, 40), (3, 3, 41)]
 
 
 def rel(a, b):
@@ -69,14 +71,18 @@ def test_order1_apply_repeats(ip, oracle, dim, n, factor):
         assert np.array_equal(s.mult(x), y)
 
 
+# 3D: 162 cells (direction in the apply) to 215,622 (two pairs per thread); 279,936 and 584,016 cells
+# take four pairs per thread, the first with both sums folded, the second with p.Ap added by a kernel in
+# between and r.z folded; 2D 361,250 cells likewise four pairs
 @pytest.mark.parametrize("dim,n,iters", [(2, 4, 1), (2, 4, 2), (2, 30, 7), (3, 3, 8), (3, 12, 9), (3, 27, 12),
-                                         (3, 33, 12)])
+                                         (3, 33, 12), (2, 425, 21), (3, 36, 12), (3, 46, 13)])
 @pytest.mark.parametrize("mixed", [False, True])
 @pytest.mark.parametrize("factor", [False, True])
 def test_coarse_cg_forms(ip, oracle, dim, n, iters, mixed, factor):
     """The order-1 Jacobi-CG with the direction formed in the apply (small meshes), as updates of their
-    own, with sums folded into the next kernel and added by a kernel in between; odd and even counts.
-    The preconditioned solve must end at the oracle's residual and take the same iterations twice."""
+    own, with one, two and four pairs per thread, with sums folded into the next kernel and added by a kernel
+    in between; odd and even counts. The preconditioned solve must end at the oracle's residual and
+    take the same iterations twice."""
     mesh = ip.Mesh.square(n, jitter=0.1, seed=5) if dim == 2 else ip.Mesh.cube(n, 0.1, 5)
     s = ip.PoissonSolver(mesh, 2)
     o = oracle.Oracle(*mesh.arrays(), 2)
