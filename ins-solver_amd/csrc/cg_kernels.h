@@ -17,21 +17,12 @@ struct Parts {
   const double* p;
   int n;
 };
-// More partials than this are added by a kernel of their own (finalize) where every block of a consumer
-// over the whole vector would read them all.
-constexpr int kFoldParts = 1024;
-
 // Scalar slots of the iteration: r.z of the last and of this iteration (they trade places), p.Ap, and
 // the step length of the direction that x still lacks.
 struct CgSlots {
   double* scal;
   int rz_old, rz_new, pap, asave;
 };
-
-// Whether a consumer of so many blocks adds so many partials itself: together they read at most 19 MB
-// from L2. 3D order-1 iteration: 236k cells 32.9 -> 29.1 us folded; 547k cells with 2136 partials read by
-// 2136 blocks 57.4 -> 58.5, by 1068 blocks 54.5.
-inline bool fold_pays(int64_t parts, int64_t blocks) { return parts * blocks <= 2400000; }
 
 // x = 0, z = p = inv b; partials of b.z. Returns their number. n is even, every vector 16-byte
 // aligned (as below).

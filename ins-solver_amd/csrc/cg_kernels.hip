@@ -312,10 +312,12 @@ void cg_update_x(int64_t n, T* x, const T* p, const CgSlots& c, hipStream_t s) {
   check("k_cg_x");
 }
 
-// FP64, constant coefficient. With more cells the gathers of two vectors per neighbour lose:
-// us per coarse iteration, update and apply / direction pass: 2D 1,800 cells 11.4 / 9.4, 65k 12.9 /
-// 10.5; 3D 3k 12.2 / 10.5, 64k 14.4 / 12.8, 132k 21.0 / 22.4, 547k 58.5 / 68.9 (two thirds of the
-// apply's waves fit beside the second set of neighbour values).
+// With more cells the gathers of two vectors per neighbour lose. us per coarse iteration, update and apply /
+// direction pass, FP64, k = 1: 2D 1,800 cells 11.4 / 9.4, 65k 12.9 / 10.5; 3D 3k 12.2 / 10.5, 64k 14.4 /
+// 12.8, 132k 21.0 / 22.4, 547k 58.5 / 68.9 (two thirds of the apply's waves fit beside the second set of
+// neighbour values). The other forms cross later. Per two iterations (FP32: one), 3D 93,750 cells:
+// FP64 32.0 / 30.0, with a coefficient 34.0 / 32.4, FP32 13.6 / 11.5, with a coefficient 14.7 / 12.5; 162,000:
+// 41.6 / 43.1, 46.4 / 45.9, 16.3 / 14.8, 17.0 / 18.1; 2D 260,642: 40.7 / 38.8, 44.7 / 43.4, 16.2 / 15.0, 16.7 / 15.6.
 bool p1_direction_pays(const MeshView& m) {
   return m.nbc && m.E <= (m.dim == 2 ? int64_t(1) << 18 : (int64_t(1) << 16) + (int64_t(1) << 15));
 }

@@ -206,13 +206,6 @@ k_pcg_direction(int64_t n2, double2* __restrict__ p, const double2* __restrict__
   p[i] = pi;
 }
 
-// Blocks of a stream of n2 pairs: few enough partials to fold while a thread has at most two pairs.
-int stream_blocks(int64_t n2) {
-  const int64_t one = (n2 + kBlock - 1) / kBlock;
-  if (one <= 2 * kFoldParts) return (int)std::max<int64_t>(1, std::min<int64_t>(one, kFoldParts));
-  return (int)std::min<int64_t>((one + 1) / 2, kRedBlocks);
-}
-
 }  // namespace
 
 void pcg_start(double* st, hipStream_t s) {
@@ -222,7 +215,7 @@ void pcg_start(double* st, hipStream_t s) {
 
 int pcg_update_jacobi(int64_t n, double* x, double* r, double* z, const double* p, const double* Ap,
                       const double* inv, Parts pap, double* st, const PcgTurn& t, double* partial, hipStream_t s) {
-  const int nb = stream_blocks(n / 2);
+  const int nb = (int)pcg_stream_blocks(n / 2);
   auto v2 = [](const double* q) { return reinterpret_cast<const double2*>(q); };
   hipLaunchKernelGGL(k_pcg_jacobi, dim3(nb), dim3(kBlock), 0, s, n / 2, reinterpret_cast<double2*>(x),
                      reinterpret_cast<double2*>(r), reinterpret_cast<double2*>(z), v2(p), v2(Ap), v2(inv), pap,
@@ -259,13 +252,13 @@ int pcg_update_inv_mass(int np, int ncomp, int64_t E, int64_t stride, int64_t cs
 void pcg_direction(int64_t n, double* p, const double* z, int nb, const double* partial, double* st,
                    const PcgTurn& t, double tol, hipStream_t s) {
   PcgSums sums{partial, nb, nb};
-  if (nb > kFoldParts) {
+  const int64_t n2 = n / 2, blocks = (n2 + kBlock - 1) / kBlock;
+  if (!pcg_fold_pays(nb, blocks)) {
     hipLaunchKernelGGL(k_pcg_sums, dim3(1), dim3(kBlock), 0, s, sums, st + P_SUM);
     check("k_pcg_sums");
     sums = PcgSums{st + P_SUM, 1, 1};
   }
-  const int64_t n2 = n / 2;
-  hipLaunchKernelGGL(k_pcg_direction, dim3((unsigned)((n2 + kBlock - 1) / kBlock)), dim3(kBlock), 0, s, n2,
+  hipLaunchKernelGGL(k_pcg_direction, dim3((unsigned)blocks), dim3(kBlock), 0, s, n2,
                      reinterpret_cast<double2*>(p), reinterpret_cast<const double2*>(z), sums, st, t, tol);
   check("k_pcg_direction");
 }

@@ -152,7 +152,9 @@ int VecViscousSolver::apply(const double* u, double* out, double* partial) {
     launch_trace_split<double>(mv, lv, u, k, tr_.p, base_.stream_, ncomp_, cs, ts);
   else
     for (int c = 0; c < ncomp_; ++c) launch_trace<double>(mv, lv, u + c * cs, k, tr_.p + c * ts, base_.stream_);
-  // the components' cells run together
+  // the components' cells run together, and the lines are the scalar pass's. The one launch is ahead well past
+  // them: us per Jacobi iteration, component by component / one launch, order 2 235,824 cells 436 / 348, 444,528
+  // 737 / 656; order 3 34,992 464 / 229, 63,888 534 / 363; order 4 20,250 951 / 430, 41,154 1225 / 768.
   MeshView all = mv;
   all.E *= ncomp_;
   if (split_apply(all, lv, false)) {

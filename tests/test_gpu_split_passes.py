@@ -71,11 +71,12 @@ def test_order1_apply_repeats(ip, oracle, dim, n, factor):
         assert np.array_equal(s.mult(x), y)
 
 
-# 3D: 162 cells (direction in the apply) to 215,622 (two pairs per thread); 279,936 and 584,016 cells
-# take four pairs per thread, the first with both sums folded, the second with p.Ap added by a kernel in
-# between and r.z folded; 2D 361,250 cells likewise four pairs
+# 3D: 162 cells (direction in the apply) to 215,622 (two pairs per thread); 279,936 and 584,016 cells take
+# four pairs per thread and fold both sums, as 2D 361,250 does; 2D 980,000 cells fold r.z and leave p.Ap to
+# a kernel in between, 3D 795,906 leave both (two pairs). The two largest carry a mass term, which keeps the
+# number of outer iterations small.
 @pytest.mark.parametrize("dim,n,iters", [(2, 4, 1), (2, 4, 2), (2, 30, 7), (3, 3, 8), (3, 12, 9), (3, 27, 12),
-                                         (3, 33, 12), (2, 425, 21), (3, 36, 12), (3, 46, 13)])
+                                         (3, 33, 12), (2, 425, 21), (3, 36, 12), (3, 46, 13), (2, 700, 8), (3, 51, 9)])
 @pytest.mark.parametrize("mixed", [False, True])
 @pytest.mark.parametrize("factor", [False, True])
 def test_coarse_cg_forms(ip, oracle, dim, n, iters, mixed, factor):
@@ -91,6 +92,9 @@ def test_coarse_cg_forms(ip, oracle, dim, n, iters, mixed, factor):
         k = 1.0 + rng.random((s.n_cells, s.Np))
         s.set_factor(k)
         o.set_factor(k)
+    if s.n_cells > 750000:
+        s.set_mm_const(10.0 * n * n)
+        o.set_mm_const(10.0 * n * n)
     s.set_pmg([2, 1], coarse_iters=iters)
     s.set_precision(ip.PRECISION_MIXED if mixed else ip.PRECISION_FP64)
     s.set_tol_and_iter(1e-9, 0.0, 2000)
