@@ -491,9 +491,11 @@ __device__ __forceinline__ void p1_store(T* o, int64_t stride, int64_t e, const 
   }
 }
 
-// Two-bit field c of w (c < 6 in 2D, < 24 in 3D), by 32-bit shifts: v_lshrrev_b64 with its amount in the
-// last VGPR of the wave's allocation (v79 of 80) took wrong amounts in about one wave of 2000 here
-// (2D order-1 apply, 125,000 cells, other results on every launch).
+// Two-bit field c of w (c < 6 in 2D, < 24 in 3D), by 32-bit shifts. With one 64-bit shift the 2D order-1 apply
+// gave wrong results in about one wave of 2000 (125,000 cells, other ones on every launch); its v_lshrrev_b64
+// had the amount in the last VGPR of the wave's allocation (v79 of 80). That the instruction was the cause is
+// inferred: 32-bit shifts also change the register allocation. (gfx90a has this fault, and LLVM keeps such
+// amounts out of that register there.)
 template <int DIM>
 __device__ __forceinline__ int node_field(unsigned long long w, int c) {
   const unsigned lo = (unsigned)w, hi = (unsigned)(w >> 32);
