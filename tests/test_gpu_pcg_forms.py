@@ -44,6 +44,9 @@ def test_solve_ends_on_the_true_residual(ip, oracle, kind, dim, N, n):
     assert s.last_stats["fine_applies"] >= its
     y = x.copy()
     assert s.solve(b, y) and s.last_stats["iterations"] == 0 and np.array_equal(x, y)
+    # every sum has one order: the same bits again
+    y = np.zeros_like(b)
+    assert s.solve(b, y) and s.last_stats["iterations"] == its and np.array_equal(x, y)
     # a limit ends the run at its iterate, with the true residual of that iterate reported
     for limit in (1, 5, 8, 13):
         if limit >= its:
@@ -94,4 +97,6 @@ def test_vector_solve(ip, oracle, N, n, jacobi):
     assert np.abs(s.mult(u) - want).max() < (1e-12 if N < 4 else 1e-11) * np.abs(want).max()
     x = np.zeros_like(u)
     assert s.solve(u, x)
+    y = np.zeros_like(u)
+    assert s.solve(u, y) and np.array_equal(x, y)
     assert np.linalg.norm(u - o.mult_vec(np.stack(bct), x)) <= 1.01e-8 * np.linalg.norm(u)
